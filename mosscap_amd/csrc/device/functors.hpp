@@ -19,6 +19,7 @@
 
 #include "layout.hpp"
 #include "fast32.hpp"
+#include "fast64.hpp"
 #include <type_traits>
 
 namespace mh {
@@ -29,10 +30,11 @@ struct Arith;
 
 template <>
 struct Arith<double> {
-    // IEEE-correct divide and sqrt (the gfx950 f64 expansions are correctly
-    // rounded), matching glibc on the host.
-    __host__ __device__ static inline double div(double a, double b) { return a / b; }
+    // correctly rounded divide and sqrt, matching glibc on the host (fast64.hpp)
+    __host__ __device__ static inline double div(double a, double b) { return div_ieee(a, b); }
     __host__ __device__ static inline double sqrt(double a) { return __builtin_sqrt(a); }
+    // ... of an argument that is 0 or of moderate size (a speed squared, HLLC's star factor)
+    __host__ __device__ static inline double sqrt_mid(double a) { return sqrt_plain(a); }
     static constexpr double weno_eps = 1e-36;  // Reconstruct.hpp:237-239
 };
 
@@ -41,6 +43,7 @@ struct Arith<float> {
     // Precision form: hardware reciprocal / sqrt (about 1 ulp).
     __device__ static inline float div(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
     __device__ static inline float sqrt(float a) { return __builtin_amdgcn_sqrtf(a); }
+    __device__ static inline float sqrt_mid(float a) { return sqrt(a); }
     static constexpr float weno_eps = 1e-15f;  // single-precision value, Reconstruct.hpp:235-236
 };
 
@@ -63,6 +66,7 @@ __host__ __device__ inline float sign1(float a) { return __builtin_copysignf(1.0
 template <typename T>
 struct EosT {
     T gamma;
+    Recip<T> gm1{gamma - T(1)};  // the divisor of p / (gamma - 1)
 };
 
 // The FP32 functors take the EOS constants rounded once from FP64 (fast32.hpp).
@@ -88,7 +92,7 @@ __host__ __device__ inline EosT<float> make_eos<float>(double gamma) {
 template <int NumDim, typename T, typename WType>
 __host__ __device__ inline T sound_speed(const T gamma, const WType& w) {
     using P = Prim<NumDim>;
-    return Arith<T>::sqrt(Arith<T>::div(gamma * w[P::Pres], w[P::Rho]));
+    return Arith<T>::sqrt_mid(Arith<T>::div(gamma * w[P::Pres], w[P::Rho]));
 }
 
 // cons_to_prim, Eos.hpp:61-79
@@ -113,7 +117,7 @@ __host__ __device__ inline void cons_to_prim(const T gamma, const QType& q, WTyp
 
 // prim_to_cons, Eos.hpp:81-99
 template <int NumDim, typename T, typename WType, typename QType>
-__host__ __device__ inline void prim_to_cons(const T gamma, const WType& w, QType& q) {
+__host__ __device__ inline void prim_to_cons(const EosT<T>& eos, const WType& w, QType& q) {
     using P = Prim<NumDim>;
     using C = Cons<NumDim>;
     q[C::Rho] = w[P::Rho];
@@ -128,13 +132,13 @@ __host__ __device__ inline void prim_to_cons(const T gamma, const WType& w, QTyp
         v2_sum += square(w[P::Vz]);
     }
     const T e_kin = T(0.5) * w[P::Rho] * v2_sum;
-    const T e_int = Arith<T>::div(w[P::Pres], gamma - T(1));
+    const T e_int = eos.gm1.div(w[P::Pres]);
     q[C::Ene] = e_int + e_kin;
 }
 
 // prim_to_flux, Eos.hpp:101-131
 template <int Axis, int NumDim, typename T, typename WType, typename FType>
-__host__ __device__ inline void prim_to_flux(const T gamma, const WType& w, FType& f) {
+__host__ __device__ inline void prim_to_flux(const EosT<T>& eos, const WType& w, FType& f) {
     using P = Prim<NumDim>;
     using C = Cons<NumDim>;
     constexpr int IV1 = Velocity<Axis, NumDim>();
@@ -154,7 +158,7 @@ __host__ __device__ inline void prim_to_flux(const T gamma, const WType& w, FTyp
     }
     e_kin *= T(0.5) * w[P::Rho];
     f[IM1] += w[P::Pres];
-    const T e_tot = Arith<T>::div(w[P::Pres], gamma - T(1)) + e_kin;
+    const T e_tot = eos.gm1.div(w[P::Pres]) + e_kin;
     f[C::Ene] = (e_tot + w[P::Pres]) * w[IV1];
 }
 
@@ -214,7 +218,9 @@ __host__ __device__ inline void reconstruct_stencil(const S& s, T& wL, T& wR) {
         wR = r;
     } else if constexpr (std::is_same_v<T, float>) {  // precision form
         weno5z_f32(s, wL, wR);
-    } else {  // WENO5-Z (Borges et al. 2008), 217-274
+    } else if constexpr (std::is_same_v<T, double>) {  // the drop-in
+        weno5z_f64(s, wL, wR);
+    } else {  // WENO5-Z (Borges et al. 2008), 217-274, for dual numbers
         constexpr T b0c = T(13) / T(12);
         constexpr T b1c = T(0.25);
         const T sm2 = s(-2), sm1 = s(-1), s0 = s(0), sp1 = s(1), sp2 = s(2);
@@ -280,10 +286,10 @@ __host__ __device__ inline void riemann_flux(const EosT<T>& eos, const WL& wL, c
     } else if constexpr (rs == RiemannSolver::Rusanov) {  // 22-46
         const T vL = wL[IV];
         const T vR = wR[IV];
-        prim_to_cons<NumDim>(gamma, wL, qL);
-        prim_to_cons<NumDim>(gamma, wR, qR);
-        prim_to_flux<Axis, NumDim>(gamma, wL, fL);
-        prim_to_flux<Axis, NumDim>(gamma, wR, fR);
+        prim_to_cons<NumDim>(eos, wL, qL);
+        prim_to_cons<NumDim>(eos, wR, qR);
+        prim_to_flux<Axis, NumDim>(eos, wL, fL);
+        prim_to_flux<Axis, NumDim>(eos, wR, fR);
         const T csL = sound_speed<NumDim>(gamma, wL);
         const T csR = sound_speed<NumDim>(gamma, wR);
         const T max_c = T(0.5) * (csL + sabs(vL) + csR + sabs(vR));
@@ -300,10 +306,10 @@ __host__ __device__ inline void riemann_flux(const EosT<T>& eos, const WL& wL, c
         // exactly as Riemann.hpp:60 does.
         const T sR = smax(-tiny, smax(wL[IV] + csL, wL[IV] + csR));
         const T sM = Arith<T>::div(T(1), sR - sL);
-        prim_to_cons<NumDim>(gamma, wL, qL);
-        prim_to_cons<NumDim>(gamma, wR, qR);
-        prim_to_flux<Axis, NumDim>(gamma, wL, fL);
-        prim_to_flux<Axis, NumDim>(gamma, wR, fR);
+        prim_to_cons<NumDim>(eos, wL, qL);
+        prim_to_cons<NumDim>(eos, wR, qR);
+        prim_to_flux<Axis, NumDim>(eos, wL, fL);
+        prim_to_flux<Axis, NumDim>(eos, wR, fR);
 #pragma unroll
         for (int i = 0; i < n_hydro; ++i) {
             flux[i] = sM * (sR * fL[i] - sL * fR[i] + sR * sL * (qR[i] - qL[i]));
@@ -314,8 +320,8 @@ __host__ __device__ inline void riemann_flux(const EosT<T>& eos, const WL& wL, c
         const T csL = sound_speed<NumDim>(gamma, wL);
         const T csR = sound_speed<NumDim>(gamma, wR);
         constexpr T tiny = T(1e-20);
-        prim_to_cons<NumDim>(gamma, wL, qL);
-        prim_to_cons<NumDim>(gamma, wR, qR);
+        prim_to_cons<NumDim>(eos, wL, qL);
+        prim_to_cons<NumDim>(eos, wR, qR);
 
         const T pL = wL[P::Pres];
         const T pR = wR[P::Pres];
@@ -323,8 +329,8 @@ __host__ __device__ inline void riemann_flux(const EosT<T>& eos, const WL& wL, c
         const T cs_avg = T(0.5) * (csL + csR);
         const T p_mid = T(0.5) * (pL + pR + (wL[IV] - wR[IV]) * rho_avg * cs_avg);
         const T g_fac = Arith<T>::div(gamma + T(1), T(2) * gamma);
-        const T cLstar = (p_mid <= pL) ? T(1) : Arith<T>::sqrt(T(1) + g_fac * (Arith<T>::div(p_mid, pL) - T(1)));
-        const T cRstar = (p_mid <= pR) ? T(1) : Arith<T>::sqrt(T(1) + g_fac * (Arith<T>::div(p_mid, pR) - T(1)));
+        const T cLstar = (p_mid <= pL) ? T(1) : Arith<T>::sqrt_mid(T(1) + g_fac * (Arith<T>::div(p_mid, pL) - T(1)));
+        const T cRstar = (p_mid <= pR) ? T(1) : Arith<T>::sqrt_mid(T(1) + g_fac * (Arith<T>::div(p_mid, pR) - T(1)));
 
         const T aL = wL[IV] - csL * cLstar;
         const T aR = wR[IV] + csR * cRstar;
@@ -337,9 +343,9 @@ __host__ __device__ inline void riemann_flux(const EosT<T>& eos, const WL& wL, c
         const T tR = pR + vxR * qR[IM];
         const T mL = wL[P::Rho] * vxL;
         const T mR = -(wR[P::Rho] * vxR);
-        const T inv_m = mL + mR;
-        const T aM = Arith<T>::div(tL - tR, inv_m);
-        const T cp = smax(Arith<T>::div(mL * tR + mR * tL, inv_m), T(0));
+        const Recip<T> inv_m(mL + mR);
+        const T aM = inv_m.div(tL - tR);
+        const T cp = smax(inv_m.div(mL * tR + mR * tL), T(0));
 
         vxL = wL[IV] - bM;
         vxR = wR[IV] - bP;
@@ -362,18 +368,14 @@ __host__ __device__ inline void riemann_flux(const EosT<T>& eos, const WL& wL, c
         fL[C::Ene] = qL[C::Ene] * vxL + pL * wL[IV];
         fR[C::Ene] = qR[C::Ene] * vxR + pR * wR[IV];
 
-        T sL, sR, sM;
-        if (aM >= T(0)) {
-            const T d = aM - bM;
-            sL = Arith<T>::div(aM, d);
-            sR = T(0);
-            sM = Arith<T>::div(-bM, d);
-        } else {
-            const T d = bP - aM;
-            sL = T(0);
-            sR = Arith<T>::div(-aM, d);
-            sM = Arith<T>::div(bP, d);
-        }
+        // the side's operands are selected before the two divisions, so that a
+        // wavefront with both signs of aM divides once
+        const bool left = aM >= T(0);
+        const Recip<T> d(left ? aM - bM : bP - aM);
+        const T sK = d.div(left ? aM : -aM);
+        const T sM = d.div(left ? -bM : bP);
+        const T sL = left ? sK : T(0);
+        const T sR = left ? T(0) : sK;
 #pragma unroll
         for (int v = 0; v < n_hydro; ++v) {
             flux[v] = sL * fL[v] + sR * fR[v];
