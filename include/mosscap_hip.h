@@ -67,8 +67,8 @@ typedef struct {
     int32_t precision_form; /* MH_FORM_* */
     int32_t span_rows;      /* rows marched per wavefront in 2-D (the rows are split into
                              * ceil(ny / span_rows) spans whose heights differ by at most
-                             * one); <= 0: the default layout, the most spans whose
-                             * wavefronts fit the GPU in one round at 4 per SIMD */
+                             * one); <= 0: the default layout, chosen by grid size so
+                             * that every SIMD holds the same number of wavefronts */
     float rho_floor;        /* FP32C positivity floors on the reconstruction input (cells and
                              * faces) and on each stage's new state (a cell below rho_floor is
                              * put at rest at (rho_floor, p_floor); one below p_floor gets its

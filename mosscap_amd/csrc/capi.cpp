@@ -105,7 +105,7 @@ int mh_create(const mh_grid_size* sz, double dx, const mh_grid_loc* loc, const m
     c->ncells = ncells;
     c->nvals = ncells * nvar;
     c->strips = (nx + kStripOut - 1) / kStripOut;
-    c->nspans = march_spans(c->opt.span_rows, c->strips, ny, nz);
+    c->nspans = march_spans(c->opt.span_rows, c->strips, ny, nz, !c->fp32c());
 
     hipError_t e = hipGetDevice(&c->device);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
@@ -590,7 +590,7 @@ int mh_autotune(mh_ctx* ctx, int32_t steps, const int32_t* candidates, int32_t* 
     const int nz = ctx->nd > 2 ? ctx->sz.zc - 2 * ctx->sz.ng : 1;
     for (int k = 0; cand[k] != 0 && e == hipSuccess; ++k) {
         if (cand[k] > ny && k > 0) continue;
-        ctx->nspans = march_spans(cand[k], ctx->strips, ny, nz);
+        ctx->nspans = march_spans(cand[k], ctx->strips, ny, nz, !ctx->fp32c());
         for (int g = 0; g < 3; ++g) {  // graphs bake the launch shape in
             if (ctx->graph[g]) hipGraphExecDestroy(ctx->graph[g]);
             ctx->graph[g] = nullptr;

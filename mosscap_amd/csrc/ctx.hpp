@@ -23,17 +23,11 @@ inline bool valid_bc(int32_t b) { return b >= 0 && b <= 6; }
 
 // Spans per plane of the 2-D march (each wavefront marches one span of a
 // strip; the ny rows are split into spans whose heights differ by at most one
-// row). rows > 0: spans of about that many rows. rows <= 0, the default
-// layout: the most spans whose wavefronts all fit 1024 SIMDs at 4 waves each
-// (every SIMD then holds 4 wavefronts and none waits for a second round) with
-// at least 8 rows each (the y halo costs 2R+2 rows per span), and spans of at
-// most 32 rows when even that needs several rounds.
-inline int march_spans(int rows, int strips, int ny, int nz) {
+// row). rows > 0: spans of about that many rows; rows <= 0: split_marches,
+// with a prologue (halo rows, first y face) worth 1.75 rows.
+inline int march_spans(int rows, int strips, int ny, int nz, bool fp64) {
     if (rows > 0) return (ny + rows - 1) / rows;
-    const int64_t fill = 4096 / ((int64_t)strips * nz);
-    const int64_t n = fill < ny / 8 ? fill : ny / 8;
-    const int64_t floor32 = (ny + 31) / 32;
-    return (int)(n > floor32 ? n : (floor32 > 0 ? floor32 : 1));
+    return split_marches((int64_t)strips * nz, ny, 1.75, fp64);
 }
 
 // Message returned by mh_last_error(NULL) (functions without a context).
