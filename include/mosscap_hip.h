@@ -332,14 +332,15 @@ int mh_batch_offsets(const mh_batch* b, int64_t* offsets);
 int mh_batch_upload(mh_batch* b, const double* q_host);
 int mh_batch_download(mh_batch* b, double* q_host);
 int mh_batch_fill_bcs(mh_batch* b);
-/* nsteps steps of every problem. mode 0: one persistent launch per stage
+/* nsteps steps of every problem. mode 0: one launch per stage
  * covering all problems (work list of 62-cell segments); mode 1: one launch
  * per problem and stage (the comparison baseline). With use_graph, each step
  * replays a captured HIP graph. Steps past max_time have dt = 0. */
 int mh_batch_run(mh_batch* b, int64_t nsteps, double max_cfl, double max_time, int32_t mode, int32_t use_graph);
 /* Per-problem clock and last dt (nprob values each; either may be NULL). */
 int mh_batch_times(mh_batch* b, double* times, double* last_dt);
-/* Persistent grid size in wavefronts (0 = built-in default), and an
+/* Grid size of a stage in wavefronts (0 = the default, one per 62-cell segment; fewer
+ * walk the work list), and an
  * autotuner that times candidate sizes (0-terminated list of waves per CU,
  * NULL = built-in) over `steps` steps, restores the state and keeps the best. */
 int mh_batch_set_waves(mh_batch* b, int32_t waves);

@@ -2,7 +2,7 @@
 //
 // Layout: problem p owns a contiguous block [3][xc_p] (xc_p = n_p + 2 ng) at
 // element offset base_p; the blocks are packed back to back. A host-built work
-// list holds one item per (problem, 62-cell segment). One persistent launch
+// list holds one item per (problem, 62-cell segment). One launch
 // per stage walks the list (wave w takes items w, w + grid, ...), so every
 // wavefront does equal work whatever the length mix; each problem keeps its
 // own dx, dt and time, and the CFL max is reduced per problem with atomics.
@@ -35,13 +35,19 @@ struct BatchGrid {
     double max_cfl = 0.0, max_time = 0.0;
 };
 
+// Element i of an array that the running launch does not write, i the same in
+// every lane: a scalar load, which leaves the vector loads in flight alone.
+template <class T>
+__device__ inline T uniform_load(const T* p, int i) {
+    return *(const __attribute__((address_space(4))) T*)(p + i);
+}
+
 // A problem's next dt from its CFL max and clock (compute_dt_impl's
 // dx / max(a) times max_cfl, clamped to end exactly at max_time with the
-// reference's nextafter loop). Reads only.
-__device__ inline double batch_next_dt(const BatchArrays& b, int pr, double max_cfl, double max_time) {
-    const double amax = __builtin_bit_cast(double, b.amax[pr]);
-    double dt = (b.dx[pr] / amax) * max_cfl;
-    const double t = b.time[pr];
+// reference's nextafter loop).
+__device__ inline double batch_next_dt(unsigned long long amax_bits, double dx, double t, double max_cfl,
+                                       double max_time) {
+    double dt = (dx / __builtin_bit_cast(double, amax_bits)) * max_cfl;
     if (t + dt >= max_time) {
         dt = max_time - t;
         while (t + dt < max_time) dt = nextafter(dt, 1.7976931348623157e308);
@@ -49,10 +55,12 @@ __device__ inline double batch_next_dt(const BatchArrays& b, int pr, double max_
     return dt;
 }
 
-// Each wave walks its items with the next item's loads issued before the
+// Loop = false: one item per wave (the grid covers the list). Loop = true:
+// each wave walks its items with the next item's loads issued before the
 // current item's arithmetic (the item carries the block offset and length,
-// so those loads wait for nothing but the item itself).
-template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS>
+// so those loads wait for nothing but the item itself, which comes as a
+// scalar load).
+template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS, bool Loop>
 __device__ inline void batch_stage(const BatchGrid& g, const typename Form::Ptrs& p, const BatchArrays& b) {
     using T = typename Form::real;
     constexpr int ORD = stencil_order(R);
@@ -61,32 +69,41 @@ __device__ inline void batch_stage(const BatchGrid& g, const typename Form::Ptrs
     const int virt = Form::kVirtualGhosts ? g.virt : 0;
     const bool per = g.per != 0;
     unsigned int hits = 0;
-    int it = blockIdx.x;
-    int4 w = it < g.nitems ? b.items[it] : make_int4(0, 0, 0, 0);
+    // Consecutive items go to one XCD: a segment's 62 cells are not a whole
+    // number of cache lines, so its neighbours read and write the lines at its
+    // ends too.
+    int it = (int)xcd_remap(blockIdx.x, gridDim.x);
+    using Item = __attribute__((ext_vector_type(4))) int;
+    const Item* items = reinterpret_cast<const Item*>(b.items);
+    Item w = uniform_load(items, it < g.nitems ? it : 0);
     SegRaw<Form> cur;
     if (it < g.nitems) seg_load<Form, R>(p, g.kind, w.z, w.w, g.ng, w.w - 2 * g.ng, w.y, virt, per, cur);
     for (; it < g.nitems; it += gridDim.x) {
-        const int nit = it + (int)gridDim.x;
-        int4 wn = w;
-        SegRaw<Form> nxt = cur;
-        if (nit < g.nitems) {
-            wn = b.items[nit];
-            seg_load<Form, R>(p, g.kind, wn.z, wn.w, g.ng, wn.w - 2 * g.ng, wn.y, virt, per, nxt);
-        }
         const int pr = w.x, i0 = w.y, base = w.z, xc = w.w;
         double dt_step;
         if (g.fin == 1) {
-            dt_step = batch_next_dt(b, pr, g.max_cfl, g.max_time);
-            if (i0 == g.ng && lane == 0) b.dt[pr] = dt_step;
+            // (this launch writes neither the CFL maxima nor the clocks)
+            dt_step = batch_next_dt(uniform_load(b.amax, pr), uniform_load(b.dx, pr), uniform_load(b.time, pr),
+                                    g.max_cfl, g.max_time);
         } else {
-            dt_step = b.dt[pr];
-            if (g.fin == 2 && i0 == g.ng && lane == 0) {
+            dt_step = uniform_load(b.dt, pr);
+        }
+        const double dx = uniform_load(b.dx, pr);
+        const int nit = it + (int)gridDim.x;
+        SegRaw<Form> nxt = cur;
+        if (Loop && nit < g.nitems) {
+            w = uniform_load(items, nit);
+            seg_load<Form, R>(p, g.kind, w.z, w.w, g.ng, w.w - 2 * g.ng, w.y, virt, per, nxt);
+        }
+        if (i0 == g.ng && lane == 0) {  // the wave with the problem's first segment
+            if (g.fin == 1) b.dt[pr] = dt_step;
+            if (g.fin == 2) {
                 b.time[pr] = b.time[pr] + dt_step;
                 b.amax[pr] = 0ull;
             }
         }
         const T dt = (T)dt_step;
-        const T dtdx = dt / (T)b.dx[pr];
+        const T dtdx = dt / (T)dx;
         double amax = 0.0;
         seg_compute<Form, R, SL, RS>(p, g.kind, g.reduce_dt, base, xc, g.ng, xc - 2 * g.ng, i0, dtdx, dt, lds, amax,
                                      hits, cur);
@@ -94,7 +111,7 @@ __device__ inline void batch_stage(const BatchGrid& g, const typename Form::Ptrs
             const uint64_t m = wave_max_u64(__builtin_bit_cast(uint64_t, amax));
             if (lane == 0) atomicMax(&b.amax[pr], (unsigned long long)m);
         }
-        w = wn;
+        if constexpr (!Loop) break;
         cur = nxt;
     }
     if (p.floor_hits != nullptr) {

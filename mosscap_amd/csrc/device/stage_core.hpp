@@ -595,11 +595,20 @@ __device__ inline void seg_load(const typename Form::Ptrs& p, int kind, int base
     const int h_entry = lane < ORD ? lane : kWave + lane;
     const int h_col = virt ? copy_ghost_source(min(i0 - 1 - ORD + h_entry, xc - 1), nx, ng, per)
                            : min(i0 - 1 - ORD + h_entry, xc - 1);
+    // every load is issued before anything waits for one: no branch between
+    // them depends on, or copies, a loaded value
 #pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        s.q[v] = Form::get(p.qs, base + v * xc + c_ld);
-        s.qn[v] = Form::needs_qn(kind) ? Form::get(p.qn, base + v * xc + c_ld) : s.q[v];
-        if (ORD > 0 && halo_lane) s.qh[v] = Form::get(p.qs, base + v * xc + h_col);
+    for (int v = 0; v < NV; ++v) s.q[v] = Form::get(p.qs, base + v * xc + c_ld);
+    if (ORD > 0 && halo_lane) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) s.qh[v] = Form::get(p.qs, base + v * xc + h_col);
+    }
+    if (Form::needs_qn(kind)) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) s.qn[v] = Form::get(p.qn, base + v * xc + c_ld);
+    } else {  // the stage kinds that do not read Q^n
+#pragma unroll
+        for (int v = 0; v < NV; ++v) s.qn[v] = typename Form::raw{};
     }
 }
 

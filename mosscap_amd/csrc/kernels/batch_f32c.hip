@@ -2,7 +2,7 @@
 // error-free transforms pin contraction off themselves).
 #define MH_STAGE_WAVES_PER_EU 1
 // 5 waves per SIMD fit without spills with the next item's loads in flight
-// (96 VGPRs); the 4096-problem ensemble is fastest at 20 waves per CU.
+// (96 VGPRs) in the looping stage; of its grids 20 waves per CU are fastest.
 #define MH_BATCH_WAVES_PER_EU 5
 #include "batch_inst.hpp"
 

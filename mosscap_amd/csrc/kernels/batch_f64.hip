@@ -10,7 +10,7 @@ __global__ void batch_finalize_kernel(int nprob, double max_cfl, double max_time
                                       double* dt_out) {
     const int pr = blockIdx.x * blockDim.x + threadIdx.x;
     if (pr >= nprob) return;
-    const double dt = batch_next_dt(b, pr, max_cfl, max_time);
+    const double dt = batch_next_dt(b.amax[pr], b.dx[pr], b.time[pr], max_cfl, max_time);
     const double t = b.time[pr];
     dt_out[pr] = dt;
     b.amax[pr] = 0ull;

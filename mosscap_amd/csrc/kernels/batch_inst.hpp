@@ -8,16 +8,16 @@
 
 namespace mh {
 
-// Occupancy the register allocator must allow for the persistent stage
-// (waves per SIMD); the autotuner picks how many of them to launch.
+// Occupancy the register allocator must allow for the looping stage (waves per
+// SIMD); the one without the loop needs far fewer registers.
 #ifndef MH_BATCH_WAVES_PER_EU
 #define MH_BATCH_WAVES_PER_EU 1
 #endif
 
-template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS>
+template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS, bool Loop>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MH_BATCH_WAVES_PER_EU))) void batch_stage_kernel(
     BatchGrid g, typename Form::Ptrs p, BatchArrays b) {
-    batch_stage<Form, R, SL, RS>(g, p, b);
+    batch_stage<Form, R, SL, RS, Loop>(g, p, b);
 }
 
 template <class Form>
@@ -47,12 +47,12 @@ __global__ __launch_bounds__(256) void batch_cfl_kernel(typename Form::Planes q,
 template <class Form>
 struct BatchPick {
     using Fn = void (*)(BatchGrid, typename Form::Ptrs, BatchArrays);
-    template <Reconstruction R, SlopeLimiter SL>
+    template <Reconstruction R, SlopeLimiter SL, bool Loop>
     static Fn pick(RiemannSolver rs) {
         switch (rs) {
-            case RiemannSolver::Rusanov: return batch_stage_kernel<Form, R, SL, RiemannSolver::Rusanov>;
-            case RiemannSolver::Hll: return batch_stage_kernel<Form, R, SL, RiemannSolver::Hll>;
-            default: return batch_stage_kernel<Form, R, SL, RiemannSolver::Hllc>;
+            case RiemannSolver::Rusanov: return batch_stage_kernel<Form, R, SL, RiemannSolver::Rusanov, Loop>;
+            case RiemannSolver::Hll: return batch_stage_kernel<Form, R, SL, RiemannSolver::Hll, Loop>;
+            default: return batch_stage_kernel<Form, R, SL, RiemannSolver::Hllc, Loop>;
         }
     }
 };
@@ -61,7 +61,10 @@ template <class Form>
 hipError_t launch_batch_stage_impl(const Schemes& s, const BatchGrid& g, int grid, const typename Form::Ptrs& p,
                                    const BatchArrays& b, hipStream_t st) {
     if (g.nitems < 1 || grid < 1 || g.ng < min_ghost_cells(s.recon)) return hipErrorInvalidValue;
-    auto pick = [&]<Reconstruction R, SlopeLimiter SL>() { return BatchPick<Form>::template pick<R, SL>(s.solver); };
+    auto pick = [&]<Reconstruction R, SlopeLimiter SL>() {
+        return grid >= g.nitems ? BatchPick<Form>::template pick<R, SL, false>(s.solver)
+                                : BatchPick<Form>::template pick<R, SL, true>(s.solver);
+    };
     auto fn = pick_scheme<Form>(s, pick);
     hipLaunchKernelGGL(fn, dim3((unsigned)grid), dim3(kWave), 0, st, g, p, b);
     return hipGetLastError();
