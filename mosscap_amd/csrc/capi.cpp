@@ -104,8 +104,10 @@ int mh_create(const mh_grid_size* sz, double dx, const mh_grid_loc* loc, const m
     }
     c->ncells = ncells;
     c->nvals = ncells * nvar;
-    c->strips = (nx + kStripOut - 1) / kStripOut;
-    c->nspans = march_spans(c->opt.span_rows, c->strips, ny, nz, !c->fp32c());
+    const MarchColumns cols = march_columns(nx, nz, num_dim, recon, !c->fp32c());
+    c->strips = cols.strips;
+    c->flat = cols.flat;
+    c->nspans = march_spans(c->opt.span_rows, c->strips, ny, num_dim, !c->fp32c());
 
     hipError_t e = hipGetDevice(&c->device);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
@@ -587,10 +589,9 @@ int mh_autotune(mh_ctx* ctx, int32_t steps, const int32_t* candidates, int32_t* 
     if (e == hipSuccess) e = hipEventCreate(&a);
     if (e == hipSuccess) e = hipEventCreate(&b);
     const int ny = ctx->nd > 1 ? ctx->sz.yc - 2 * ctx->sz.ng : 1;
-    const int nz = ctx->nd > 2 ? ctx->sz.zc - 2 * ctx->sz.ng : 1;
     for (int k = 0; cand[k] != 0 && e == hipSuccess; ++k) {
         if (cand[k] > ny && k > 0) continue;
-        ctx->nspans = march_spans(cand[k], ctx->strips, ny, nz, !ctx->fp32c());
+        ctx->nspans = march_spans(cand[k], ctx->strips, ny, ctx->nd, !ctx->fp32c());
         for (int g = 0; g < 3; ++g) {  // graphs bake the launch shape in
             if (ctx->graph[g]) hipGraphExecDestroy(ctx->graph[g]);
             ctx->graph[g] = nullptr;

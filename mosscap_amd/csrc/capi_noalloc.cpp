@@ -131,7 +131,7 @@ int mh_step_noalloc(const mh_grid_size* sz, double dx, const mh_boundaries* bdry
     // the stages: Q^n stays in q_in; intermediate states rotate through the
     // two scratch states; the last stage writes q_out
     const int strips = (nx + kStripOut - 1) / kStripOut;
-    const int nspans = march_spans(0, strips, ny, 1, true);
+    const int nspans = march_spans(0, strips, ny, 2, true);
     const int ns = num_stages(sch.stepper);
     const double* in = q_in;
     for (int s = 0; s < ns && e == hipSuccess; ++s) {

@@ -21,13 +21,14 @@ inline int stage_kind(TimeStepScheme ts, int stage) {
 
 inline bool valid_bc(int32_t b) { return b >= 0 && b <= 6; }
 
-// Spans per plane of the 2-D march (each wavefront marches one span of a
+// Spans of the march (each wavefront marches one span of a
 // strip; the ny rows are split into spans whose heights differ by at most one
 // row). rows > 0: spans of about that many rows; rows <= 0: split_marches,
-// with a prologue (halo rows, first y face) worth 1.75 rows.
-inline int march_spans(int rows, int strips, int ny, int nz, bool fp64) {
+// with a prologue (halo rows, first y face) worth 1.75 rows, 3 in 3-D, where
+// the halo rows' loads weigh more.
+inline int march_spans(int rows, int strips, int ny, int nd, bool fp64) {
     if (rows > 0) return (ny + rows - 1) / rows;
-    return split_marches((int64_t)strips * nz, ny, 1.75, fp64);
+    return split_marches(strips, ny, nd > 2 ? 3.0 : 1.75, fp64);
 }
 
 // Message returned by mh_last_error(NULL) (functions without a context).
@@ -85,8 +86,8 @@ struct mh_ctx {
     // changes the state or the slots otherwise), so the next mh_run needs no
     // separate CFL pass.
     bool amax_valid = false;
-    int nspans = 1;   // spans per plane of the 2-D march (march_spans)
-    int strips = 0;
+    int nspans = 1;   // spans of the march (march_spans)
+    int strips = 0, flat = 0;  // march_columns
     std::string err;
     hipGraphExec_t graph[3] = {nullptr, nullptr, nullptr};
     // event log for mh_run_timed: (kind, start, stop); kind 0 stage, 1 ghost, 2 clock
@@ -275,6 +276,7 @@ struct mh_ctx {
         StageGrid g{sz.xc, sz.yc, sz.ng, sz.xc - 2 * sz.ng, sz.yc - 2 * sz.ng, strips, nspans, kind, reduce};
         g.zc = sz.zc;
         g.nz = sz.zc - 2 * sz.ng;
+        g.flat = flat;
         set_virt(g);
         return g;
     }

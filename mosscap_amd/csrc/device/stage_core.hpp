@@ -83,7 +83,7 @@ enum StageInst : int { kStagePlain = 0, kStageFloors = 1, kStageExtras = 2 };
 
 struct StageGrid {
     int32_t xc, yc, ng, nx, ny;
-    int32_t strips, nspans;  // 62-column strips, spans of rows per plane
+    int32_t strips, nspans;  // wavefronts side by side (2-D: 62-column strips; 3-D: of all planes), spans of rows
     int32_t kind;        // StageKind
     int32_t reduce_dt;   // fold the new state into the CFL max
     int32_t zc = 1, nz = 1;  // 3-D: planes (ghosts included) and interior planes
@@ -100,11 +100,44 @@ struct StageGrid {
     // stage reads dt from the clock.
     int32_t fin = 0;
     Clock* clock = nullptr;
+    // 3-D: slots per plane of the wavefronts' columns (march_columns), or 0
+    // when each plane has strips of its own
+    int32_t flat = 0;
 };
 
+// 3-D march: how the columns of the nz planes are dealt to wavefronts of 62
+// output lanes. Strips per plane leave the last one of each plane part empty
+// (256 columns in five strips: a fifth of the lanes idle). Flat, the planes'
+// columns, each plane's with the 1 + ORD columns that its outermost faces
+// need on either side (`flat` slots), run on from wavefront to wavefront, so
+// one may end a plane and begin the next. The FP64 march is bound by VALU
+// issue and takes the fewer wavefronts: flat unless nx is at or just below a
+// multiple of 62 (150x131x97 stage 300 -> 280 us, 128^3 338 -> 303 us). The
+// FP32C march is bound by memory as much (2.3 times its algorithmic reads
+// come from beyond L2), where a part-empty wavefront costs little and one
+// that straddles two planes reads more lines: it goes flat only to save a
+// quarter of the wavefronts (128^3: 28 % fewer, stage 160 -> 148 us; 256^3:
+// 15 % fewer, 939 -> 992 us).
+struct MarchColumns {
+    int32_t strips, flat;  // StageGrid::strips, StageGrid::flat
+};
+inline MarchColumns march_columns(int nx, int nz, int nd, Reconstruction r, bool fp64) {
+    const int per_plane = (nx + kStripOut - 1) / kStripOut;
+    if (nd < 3) return {per_plane, 0};
+    const int slots = nx + 2 * (1 + stencil_order(r));
+    const int64_t flat = ((int64_t)nz * slots + kStripOut - 1) / kStripOut, own = (int64_t)nz * per_plane;
+    if (fp64 ? flat < own : 4 * flat <= 3 * own) return {(int32_t)flat, slots};
+    return {(int32_t)own, 0};
+}
+// ... and their order: groups of wavefronts side by side (a plane's strips,
+// or kMarchGroup flat ones), within a group span by span, so that spans one
+// above the other (which read the same halo rows) run at about the same time
+// on one XCD.
+constexpr int kMarchGroup = 8;
 
-// The x-y march of one plane. ND = 2: the whole 2-D stage. ND = 3: one
-// interior z-plane per (strip, span, plane) workgroup; the z flux difference
+
+// The x-y march. ND = 2: the whole 2-D stage. ND = 3: every interior z-plane,
+// the lanes' columns as march_columns deals them; the z flux difference
 // of each cell comes from the z sweep (p.dz3) and is added after the y one,
 // as integrate_flux adds Fz after Fy (TimeStepping.cpp:22-30).
 // Inst selects what is compiled in (their addresses, operands and branches
@@ -129,25 +162,53 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
     __shared__ T xrow[NV][ROW];
 
     const int lane = threadIdx.x;
-    const uint32_t bb = xcd_remap(blockIdx.x, gridDim.x);
-    const uint32_t per_plane = (uint32_t)g.strips * (uint32_t)g.nspans;
-    const uint32_t b = bb % per_plane;
-    const int strip = (int)(b % (uint32_t)g.strips);
-    const int span = (int)(b / (uint32_t)g.strips);
-    const int i0 = g.ng + strip * kStripOut;
+    const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
+    int strip, span;
+    if constexpr (ND > 2) {
+        const uint32_t most = g.flat != 0 ? kMarchGroup : (uint32_t)((g.nx + kStripOut - 1) / kStripOut);
+        const uint32_t first = b / (most * (uint32_t)g.nspans) * most;
+        const uint32_t in_group = b % (most * (uint32_t)g.nspans);
+        const uint32_t size = min(most, (uint32_t)g.strips - first);  // the last group may be smaller
+        strip = (int)(first + in_group % size);
+        span = (int)(in_group / size);
+    } else {
+        strip = (int)(b % (uint32_t)g.strips);
+        span = (int)(b / (uint32_t)g.strips);
+    }
     // rows of this span: the ny rows split into nspans spans of equal height (+-1)
     const int j0 = g.ng + (int)(((int64_t)span * g.ny) / g.nspans);
     const int j1 = g.ng + (int)(((int64_t)(span + 1) * g.ny) / g.nspans);
-    const int c = i0 - 1 + lane;
+    // column and (3-D) plane of the lane, or of the halo entry, at position
+    // `at` along the wavefront: lanes 0 .. 63, halo entries outside
+    auto column_of = [&](int at, int& plane_idx) -> int {
+        if constexpr (ND > 2) {
+            if (g.flat != 0) {
+                const int slot = min(max(strip * kStripOut - 1 + at, 0), g.nz * g.flat - 1);
+                plane_idx = slot / g.flat;
+                return g.ng - 1 - ORD + slot % g.flat;
+            }
+            const int per_plane = (g.nx + kStripOut - 1) / kStripOut;
+            plane_idx = strip / per_plane;
+            return g.ng + (strip % per_plane) * kStripOut - 1 + at;
+        } else {
+            plane_idx = 0;
+            return g.ng + strip * kStripOut - 1 + at;
+        }
+    };
+    int kz;  // interior plane of the lane (3-D)
+    const int c = column_of(lane, kz);
     // ghosts read from their sources (StageGrid::virt; compiled for the forms that use it)
     constexpr bool kVirt = Form::kVirtualGhosts;
-    const int c_ld = (kVirt && g.virt) ? copy_ghost_source(min(c, g.xc - 1), g.nx, g.ng, g.xper) : min(c, g.xc - 1);
+    auto plane_offset = [&](int k) { return ND > 2 ? (g.ng + k) * g.xc * g.yc : 0; };
+    const int pl = plane_offset(kz);  // the lane's plane is part of its vector offset
+    // where the lane loads (an output lane stores there too: its column is interior)
+    const int c_ld =
+        pl + ((kVirt && g.virt) ? copy_ghost_source(min(c, g.xc - 1), g.nx, g.ng, g.xper) : min(c, g.xc - 1));
     // source row of row r (wave-uniform)
     auto src_row = [&](int r) { return (kVirt && g.virt) ? copy_ghost_source(r, g.ny, g.ng, g.yper) : r; };
     const int xc = g.xc;
-    // variables are [var][k][j][i]: var stride of the whole grid, then this plane's offset
+    // variables are [var][k][j][i]: var stride of the whole grid
     const int plane = g.xc * g.yc * (ND > 2 ? g.zc : 1);
-    const int pk = ND > 2 ? (g.ng + (int)(bb / per_plane)) * g.xc * g.yc : 0;
 
     // Halo columns: exchange-row entries [0, ORD) (columns left of the strip)
     // and [64+ORD, 64+2*ORD) (right of it). They are converted to primitives
@@ -205,7 +266,7 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
     const T src = T(0) * dt;
 
     T win[WIN][NV] = {};
-    const bool out_lane = lane >= 1 && lane <= kStripOut && c < g.ng + g.nx;
+    const bool out_lane = lane >= 1 && lane <= kStripOut && c >= g.ng && c < g.ng + g.nx;
 
     // Plain instance: the stage-combine operands of the next row (Q^(s) and
     // Q^n, two words per value) are loaded straight into LDS while this row
@@ -219,22 +280,21 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
     constexpr int kQnSlot = kQsRing ? 0 : 1;
     __shared__ uint32_t opnd[kDmaOps && !kQsRing ? 2 : 1][kDmaOps ? NV : 1][2][kWave];  // [Q^(s), Q^n][var][word][lane]
     // 3-D: the z flux differences of the combined row (the z sweep's output,
-    // one value per variable and interior cell; lanes outside read a clamped
-    // column that they do not use)
+    // one value per variable and interior cell; lanes outside read the
+    // column that they load, and do not use it)
     constexpr bool kDzLds = ND > 2 && kDmaOps && MH_STAGE_DZ_LDS != 0;
     constexpr int kDzWords = sizeof(T) / 4;
     __shared__ uint32_t dzo[kDzLds ? NV : 1][kDzLds ? kDzWords : 1][kWave];
-    const int c_dz = min(c, g.xc - 1);
     auto issue_operands = [&](int jr) {
         if constexpr (kDmaOps) {
-            const int row = pk + jr * xc;
+            const int row = jr * xc;
             if constexpr (kDzLds) {
                 const auto bdz = make_rsrc(p.dz3);
 #pragma unroll
                 for (int v = 0; v < NV; ++v)
 #pragma unroll
                     for (int w = 0; w < kDzWords; ++w)
-                        buf_load_lds(bdz, &dzo[v][w][0], (uint32_t)c_dz * (uint32_t)sizeof(T) + 4u * w,
+                        buf_load_lds(bdz, &dzo[v][w][0], (uint32_t)c_ld * (uint32_t)sizeof(T) + 4u * w,
                                      (uint32_t)(v * plane + row) * (uint32_t)sizeof(T));
             }
 #pragma unroll
@@ -253,24 +313,29 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
     // (the row combined next was committed ORD + 1 rows before it)
     uint32_t in_floor_bits = 0;
 
+    // this lane's halo column (with its plane): found again for every batch in
+    // 2-D, kept in 3-D, where it takes an integer division
+    auto halo_column = [&]() -> int {
+        const int idx = lane % (NH > 0 ? NH : 1);
+        int k;
+        const int col = min(column_of((idx < ORD ? idx : kWave + idx) - ORD, k), g.xc - 1);
+        return plane_offset(k) + ((kVirt && g.virt) ? copy_ghost_source(col, g.nx, g.ng, g.xper) : col);
+    };
+    const int hb_col_kept = ND > 2 ? halo_column() : 0;
     auto commit_row = [&](int r, const Raw (&q)[NV]) {
         if constexpr (NH > 0) {
             if (((r - r_first) & (HB - 1)) == 0) {  // wave-uniform: convert the halo of rows r .. r+HB-1
                 wave_lds_sync();  // the previous batch's reads are done
                 const int hb_idx = lane % NH;  // this lane's halo column
                 const int hb_row = lane / NH;  // and row offset in the batch
-                int hb_col = min(i0 - 1 - ORD + (hb_idx < ORD ? hb_idx : kWave + hb_idx), g.xc - 1);
+                const int hb_col = ND > 2 ? hb_col_kept : halo_column();
                 const int rr = r + hb_row;
                 if (hb_row < HB && rr <= r_last) {
-                    int rs = rr;
-                    if (kVirt && g.virt) {
-                        hb_col = copy_ghost_source(hb_col, g.nx, g.ng, g.xper);
-                        rs = copy_ghost_source(rr, g.ny, g.ng, g.yper);
-                    }
+                    const int rs = (kVirt && g.virt) ? copy_ghost_source(rr, g.ny, g.ng, g.yper) : rr;
                     Raw qh[NV];
                     // the lane's row goes in the vector offset (the scalar one is wave-uniform)
 #pragma unroll
-                    for (int v = 0; v < NV; ++v) qh[v] = load_qs(rs * xc + hb_col, v * plane + pk);
+                    for (int v = 0; v < NV; ++v) qh[v] = load_qs(rs * xc + hb_col, v * plane);
                     T wh[NV];
                     Form::template to_prim_nd<ND, kFloors>(p, qh, wh);
 #pragma unroll
@@ -290,7 +355,7 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
         for (int v = 0; v < NV; ++v) win[WIN - 1][v] = w[v];
     };
     auto fetch_row = [&](int r, Raw (&q)[NV]) {
-        const int base = pk + src_row(r) * xc;
+        const int base = src_row(r) * xc;
 #pragma unroll
         for (int v = 0; v < NV; ++v) q[v] = load_qs(c_ld, v * plane + base);
     };
@@ -316,7 +381,7 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
     Raw qsr[kQsRing ? ORD + 1 : 1][NV];
     auto issue_lead = [&](int r) {
         if constexpr (kDmaOps) {
-            const int base = pk + src_row(r) * xc;
+            const int base = src_row(r) * xc;
             const int sl = lead_slot(r);
 #pragma unroll
             for (int v = 0; v < NV; ++v)
@@ -388,7 +453,7 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
         // Stage-combine operands of this row: from LDS in the plain instance
         // (loaded during the previous row); otherwise loaded here or just
         // before the combine (Form::kEarlyOperands).
-        const int row = pk + j * xc;
+        const int row = j * xc;
         Raw qs_c[NV], qn_c[NV];
         auto load_operands = [&] {
 #pragma unroll
@@ -426,7 +491,7 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
         T dzr[ND > 2 && !kDzLds ? NV : 1];
         if constexpr (ND > 2 && !kDzLds) {
 #pragma unroll
-            for (int v = 0; v < NV; ++v) dzr[v] = p.dz3[v * plane + pk + j * xc + c_dz];
+            for (int v = 0; v < NV; ++v) dzr[v] = p.dz3[v * plane + j * xc + c_ld];
         }
 
         // y sweep: cell j+1, face j+1
@@ -515,8 +580,8 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
             floor_hits += (st_hit || ((in_floor_bits >> (ORD + 1)) & 1u)) ? 1u : 0u;
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
-                if constexpr (kBuf) Form::bput(bout, (uint32_t)c * ES, (uint32_t)(v * plane + row), qo[v]);
-                else Form::put(p.out, v * plane + row + c, qo[v]);
+                if constexpr (kBuf) Form::bput(bout, (uint32_t)c_ld * ES, (uint32_t)(v * plane + row), qo[v]);
+                else Form::put(p.out, v * plane + row + c_ld, qo[v]);
             }
             if (g.reduce_dt) {
                 const double a = Form::template signal_speed_nd<ND>((double)p.gamma, qo);

@@ -155,10 +155,11 @@ template <class Form>
 hipError_t launch_stage3d_impl(const Schemes& s, const StageGrid& g, const typename Form::Ptrs& p,
                                typename Form::real* dz, hipStream_t st) {
     if (g.nx < 1 || g.ny < 1 || g.nz < 1 || g.ng < min_ghost_cells(s.recon) || g.xc != g.nx + 2 * g.ng ||
-        g.yc != g.ny + 2 * g.ng || g.zc != g.nz + 2 * g.ng || g.nspans < 1 || g.nspans > g.ny ||
-        g.strips != (g.nx + kStripOut - 1) / kStripOut || !dz) {
+        g.yc != g.ny + 2 * g.ng || g.zc != g.nz + 2 * g.ng || g.nspans < 1 || g.nspans > g.ny || !dz) {
         return hipErrorInvalidValue;
     }
+    const MarchColumns cols = march_columns(g.nx, g.nz, 3, s.recon, sizeof(typename Form::real) == 8);
+    if (g.strips != cols.strips || g.flat != cols.flat) return hipErrorInvalidValue;
     using ZFn = void (*)(ZSweepGrid, typename Form::Ptrs, typename Form::real*);
     auto zpick = [&]<Reconstruction R, SlopeLimiter SL>() -> ZFn {
         switch (s.solver) {
@@ -197,7 +198,7 @@ hipError_t launch_stage3d_impl(const Schemes& s, const StageGrid& g, const typen
                        dz);
     typename Form::Ptrs pm = p;
     pm.dz3 = dz;
-    hipLaunchKernelGGL(pick_scheme<Form>(s, mpick), dim3((unsigned)(g.strips * g.nspans * g.nz)), dim3(kWave), 0, st,
+    hipLaunchKernelGGL(pick_scheme<Form>(s, mpick), dim3((unsigned)(g.strips * g.nspans)), dim3(kWave), 0, st,
                        g, pm);
     return hipGetLastError();
 }

@@ -33,7 +33,7 @@ struct Schemes {
 // rounds of as many as reside there (2 in FP64, 4 in FP32C), times a
 // wavefront's rows, times what a row takes with so many neighbours
 // (wavefronts that share a SIMD hide each other's latency: a lone FP32C row
-// takes 1.9 times its share of a full SIMD), plus a fifth of a wavefront
+// takes 1.9 times its share of a full SIMD), plus a quarter of a wavefront
 // for the last round's uneven end.
 // Measured with every split from k = 1/2 to 16 on 256^2 to 4096^2 and 64^3
 // to 256^3: the pick is within 3 % of the best split, and against a fixed
@@ -43,7 +43,7 @@ struct Schemes {
 inline int split_marches(int64_t units, int rows, double prologue, bool fp64) {
     constexpr int kSimds = 1024;
     const int resident = fp64 ? 2 : 4;
-    const double share64[] = {0.0, 1.22, 2.08}, share32[] = {0.0, 1.9, 2.4, 3.15, 4.0};  // of 1, 2, .. wavefronts
+    const double share64[] = {0.0, 1.18, 2.08}, share32[] = {0.0, 1.9, 2.4, 3.15, 4.0};  // of 1, 2, .. wavefronts
     const double* share = fp64 ? share64 : share32;
     int best = 1;
     double least = 0.0;
@@ -52,7 +52,7 @@ inline int split_marches(int64_t units, int rows, double prologue, bool fp64) {
         const int n = (int)(fit < 1 ? 1 : fit < rows ? fit : rows);
         const int64_t per_simd = (n * units + kSimds - 1) / kSimds;
         const double rounds = (double)(per_simd / resident) * share[resident] + share[per_simd % resident];
-        const double t = (rounds + 0.2) * ((double)rows / n + prologue);
+        const double t = (rounds + 0.25) * ((double)rows / n + prologue);
         if (k == 1 || t < least) {
             least = t;
             best = n;
