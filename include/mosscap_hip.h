@@ -134,9 +134,10 @@ int mh_stage(mh_ctx* ctx, int32_t stage, double dt);
  * bookkeeping, for nsteps steps (steps past max_time have dt = 0). *time and
  * *prev_output_time are read and updated. With use_graph, steps replay a
  * captured HIP graph. The first dt of a call comes from a CFL pass over the
- * state, except right after another mh_run, whose last stage left the
- * current state's maximum signal speed behind (every other call that changes
- * the state clears it). A caller that writes the state through
+ * state, except right after another mh_run, or an mh_time_step that followed
+ * mh_compute_dt, whose last stage left the current state's maximum signal speed
+ * behind (every other call that changes the state clears it); mh_compute_dt
+ * uses it too. A caller that writes the state through
  * mh_device_state outside a user_bc hook calls mh_fill_bcs afterwards, as the
  * reference's setup does, which clears it too. */
 int mh_run(mh_ctx* ctx, int64_t nsteps, double max_cfl, double* time, double max_time, double* prev_output_time,

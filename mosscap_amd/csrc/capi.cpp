@@ -111,47 +111,62 @@ int mh_create(const mh_grid_size* sz, double dx, const mh_grid_loc* loc, const m
 
     hipError_t e = hipGetDevice(&c->device);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
-    const size_t bytes64 = (size_t)c->nvals * sizeof(double);
-    const size_t bytes32 = (size_t)c->nvals * sizeof(float);
-    for (int k = 0; k < 3 && e == hipSuccess; ++k) {
-        if (c->fp32c()) {
-            e = hipMalloc(&c->qhi[k], bytes32);
-            if (e == hipSuccess) e = hipMalloc(&c->qlo[k], bytes32);
-        } else {
-            e = hipMalloc(&c->q64[k], bytes64);
+    // Buffers under 1 MiB share one allocation, cleared at once (a small grid's
+    // context is made in half the calls); a larger one has its own (planes a
+    // multiple of 2 MiB apart in one allocation made the 4096^2 FP32C step
+    // 1.6 % slower).
+    {
+        struct Want {
+            void** at;
+            size_t bytes, offset;
+            bool clear;
+        };
+        std::vector<Want> wants;
+        size_t shared = 0;
+        const auto want = [&](auto*& p, size_t bytes, bool clear) {
+            const bool own = bytes >= (size_t)1 << 20;
+            wants.push_back({reinterpret_cast<void**>(&p), bytes, own ? SIZE_MAX : shared, clear});
+            if (!own) shared = (shared + bytes + 255) / 256 * 256;
+        };
+        const size_t cells = (size_t)ncells, r = c->fp32c() ? sizeof(float) : sizeof(double);
+        const size_t state = (size_t)c->nvals * r;
+        want(c->clock, kClockBytes, true);
+        want(c->floor_hits, sizeof(unsigned int), true);
+        for (int k = 0; k < 3; ++k) {  // defined contents everywhere (ghosts of the rotating buffers included)
+            if (c->fp32c()) {
+                want(c->qhi[k], state, true);
+                want(c->qlo[k], state, true);
+            } else {
+                want(c->q64[k], state, true);
+            }
+        }
+        if (c->fp32c()) want(c->staging, (size_t)c->nvals * sizeof(double), false);
+        if (num_tracers > 0 && c->fp32c()) {
+            want(c->frx32, cells * r, false);
+            want(c->fry32, cells * r, false);
+            want(c->wtr32, cells * num_tracers * r, false);
+        } else if (num_tracers > 0) {
+            want(c->frx64, cells * r, false);
+            want(c->fry64, cells * r, false);
+            want(c->wtr64, cells * num_tracers * r, false);
+        }
+        if (num_dim == 3 && c->fp32c()) want(c->dz32, cells * 5 * r, false);
+        else if (num_dim == 3) want(c->dz64, cells * 5 * r, false);
+        const auto alloc = [&](size_t bytes) -> char* {
+            void* p = nullptr;
+            if (e == hipSuccess) e = hipMalloc(&p, bytes);
+            if (e == hipSuccess) c->buffers.push_back(p);
+            return e == hipSuccess ? static_cast<char*>(p) : nullptr;
+        };
+        char* const base = alloc(shared);
+        if (e == hipSuccess) e = hipMemsetAsync(base, 0, shared, c->stream);
+        for (const Want& w : wants) {
+            if (e != hipSuccess) break;
+            *w.at = w.offset != SIZE_MAX ? base + w.offset : alloc(w.bytes);
+            if (e == hipSuccess && w.offset == SIZE_MAX && w.clear) e = hipMemsetAsync(*w.at, 0, w.bytes, c->stream);
         }
     }
-    if (e == hipSuccess && c->fp32c()) e = hipMalloc(&c->staging, bytes64);
-    if (e == hipSuccess && num_tracers > 0) {
-        const size_t n = (size_t)ncells;
-        if (c->fp32c()) {
-            e = hipMalloc(&c->frx32, n * sizeof(float));
-            if (e == hipSuccess) e = hipMalloc(&c->fry32, n * sizeof(float));
-            if (e == hipSuccess) e = hipMalloc(&c->wtr32, n * num_tracers * sizeof(float));
-        } else {
-            e = hipMalloc(&c->frx64, n * sizeof(double));
-            if (e == hipSuccess) e = hipMalloc(&c->fry64, n * sizeof(double));
-            if (e == hipSuccess) e = hipMalloc(&c->wtr64, n * num_tracers * sizeof(double));
-        }
-    }
-    if (e == hipSuccess && num_dim == 3) {
-        const size_t n = (size_t)ncells * 5;
-        if (c->fp32c()) e = hipMalloc(&c->dz32, n * sizeof(float));
-        else e = hipMalloc(&c->dz64, n * sizeof(double));
-    }
-    if (e == hipSuccess) e = hipMalloc(&c->clock, kClockBytes);
-    if (e == hipSuccess) e = hipMalloc(&c->floor_hits, sizeof(unsigned int));
-    if (e == hipSuccess) e = hipMemsetAsync(c->clock, 0, kClockBytes, c->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(c->floor_hits, 0, sizeof(unsigned int), c->stream);
-    // defined contents everywhere (ghosts of the rotating buffers included)
-    for (int k = 0; k < 3 && e == hipSuccess; ++k) {
-        if (c->fp32c()) {
-            e = hipMemsetAsync(c->qhi[k], 0, bytes32, c->stream);
-            if (e == hipSuccess) e = hipMemsetAsync(c->qlo[k], 0, bytes32, c->stream);
-        } else {
-            e = hipMemsetAsync(c->q64[k], 0, bytes64, c->stream);
-        }
-    }
+    if (e == hipSuccess) e = hipHostMalloc(&c->clock_host, sizeof(Clock));
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) {
         g_create_error = std::string("mh_create: ") + hipGetErrorString(e);
@@ -180,7 +195,7 @@ int mh_set_user_bc(mh_ctx* ctx, mh_user_bc_fn fn, void* user) {
     if (ctx->next_stage != 0) return ctx->fail(MH_ERR_INVALID, "a step is in progress (mh_stage)");
     ctx->user_fn = fn;
     ctx->user_data = fn ? user : nullptr;
-    ctx->amax_valid = false;
+    ctx->forget_speed();
     return MH_OK;
 }
 
@@ -232,6 +247,10 @@ int mh_eos_fields(mh_ctx* ctx, int32_t which, double avg_mass, int32_t ionisatio
 int mh_device_state(mh_ctx* ctx, mh_device_view* out) {
     if (!ctx || !out) return MH_ERR_INVALID;
     const int k = ctx->view_buf >= 0 ? ctx->view_buf : ctx->cur;
+    if (ctx->view_buf < 0) {
+        ctx->exposed = true;
+        ctx->forget_speed();
+    }
     *out = mh_device_view{};
     out->precision_form = ctx->opt.precision_form;
     out->num_values = ctx->nvals;
@@ -260,10 +279,9 @@ static bool in_place(const mh_ctx* c, const double* q) {
         return false;
     }
     const size_t offset = (size_t)((const char*)q - (const char*)base), bytes = (size_t)c->nvals * sizeof(double);
-    for (int k = 0; k < 3; ++k)
-        if (base == (hipDeviceptr_t)c->qhi[k] || base == (hipDeviceptr_t)c->qlo[k]) return false;
-    return base != (hipDeviceptr_t)c->staging && offset <= size && bytes <= size - offset &&
-           (uintptr_t)q % sizeof(double) == 0;
+    for (void* own : c->buffers)
+        if (base == (hipDeviceptr_t)own) return false;
+    return offset <= size && bytes <= size - offset && (uintptr_t)q % sizeof(double) == 0;
 }
 
 // The compensated form converts between FP64 and its planes from and to the
@@ -281,7 +299,7 @@ static int upload_impl(mh_ctx* c, const double* q, hipMemcpyKind kind) {
     } else {
         if (e == hipSuccess) e = hipMemcpyAsync(c->q64[c->cur], q, bytes, kind, c->stream);
     }
-    c->amax_valid = false;
+    c->forget_speed();
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return c->hip_fail(e, "mh_upload");
     c->next_stage = 0;
@@ -313,15 +331,14 @@ int mh_download_device(mh_ctx* ctx, double* q_dev) { return download_impl(ctx, q
 int mh_fill_bcs(mh_ctx* ctx) {
     if (!ctx) return MH_ERR_INVALID;
     hipError_t e = hipSetDevice(ctx->device);
-    ctx->amax_valid = false;  // a hook may change ghost values; state written through mh_device_state
+    ctx->forget_speed();  // a hook may change ghost values; state written through mh_device_state
     if (e == hipSuccess) e = ctx->ghost(ctx->cur, ctx->cur, 0);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     return e == hipSuccess ? MH_OK : ctx->hip_fail(e, "mh_fill_bcs");
 }
 
-// Writes the clock's fields; clears the CFL slots unless `keep_max`.
-static hipError_t write_clock(mh_ctx* c, double max_cfl, double time, double max_time, double prev, double delta,
-                              bool keep_max = false) {
+// The clock's fields at the start of a run or of a step size.
+static Clock clock_fields(const mh_ctx* c, double max_cfl, double time, double max_time, double prev, double delta) {
     Clock h{};
     h.time = time;
     h.dt = 0.0;
@@ -331,8 +348,7 @@ static hipError_t write_clock(mh_ctx* c, double max_cfl, double time, double max
     h.max_cfl = max_cfl;
     h.dx = c->dx;
     h.step = c->steps;
-    const hipError_t e = hipMemcpyAsync(c->clock, &h, sizeof(Clock), hipMemcpyHostToDevice, c->stream);
-    return (e == hipSuccess && !keep_max) ? launch_clock_reset_max(c->clock, c->stream) : e;
+    return h;
 }
 
 // The tabulated EOS's abort condition (TabulatedLteH.hpp:140-142) after a
@@ -357,7 +373,7 @@ int mh_set_tabulated_eos(mh_ctx* ctx, const mh_lte_table* t) {
     if (ctx->tab_neg) hipFree(ctx->tab_neg);
     ctx->tab_neg = nullptr;
     ctx->tab_on = 0;
-    ctx->amax_valid = false;
+    ctx->forget_speed();
     ctx->drop_graphs();
     if (e != hipSuccess) return ctx->hip_fail(e, "mh_set_tabulated_eos");
     if (!t) return MH_OK;
@@ -390,7 +406,7 @@ int mh_tabulated_eos_update(mh_ctx* ctx) {
     if (!ctx->tab_on) return ctx->fail(MH_ERR_INVALID, "no tabulated EOS is installed");
     if (ctx->next_stage != 0) return ctx->fail(MH_ERR_INVALID, "a step is in progress (mh_stage)");
     hipError_t e = hipSetDevice(ctx->device);
-    ctx->amax_valid = false;
+    ctx->forget_speed();
     if (e == hipSuccess) e = ctx->tab_update(ctx->cur, ctx->cur);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) return ctx->hip_fail(e, "mh_tabulated_eos_update");
@@ -409,19 +425,27 @@ int mh_tabulated_eos_fields(mh_ctx* ctx, double* y, double* T) {
     return tab_check(ctx);
 }
 
+// One launch and one wait where the last step left the maximum signal speed of
+// the state behind (FP64 Sod 256^2: a pass over the state, two copies and
+// three clock kernels otherwise, 25 of the 72 us of a host-driven step).
 int mh_compute_dt(mh_ctx* ctx, double max_cfl, double time, double max_time, double prev_output_time,
                   double delta, double* dt_out) {
     if (!ctx || !dt_out) return MH_ERR_INVALID;
     hipError_t e = hipSetDevice(ctx->device);
-    ctx->amax_valid = false;
-    if (e == hipSuccess) e = write_clock(ctx, max_cfl, time, max_time, prev_output_time, delta);
-    if (e == hipSuccess) e = ctx->cfl_all(ctx->cur);
-    if (e == hipSuccess) e = launch_clock_finalize(ctx->clock, 0, ctx->stream);
-    Clock h{};
-    if (e == hipSuccess) e = hipMemcpyAsync(&h, ctx->clock, sizeof(Clock), hipMemcpyDeviceToHost, ctx->stream);
+    const bool keep_max = ctx->amax_valid && !ctx->exposed;
+    ctx->forget_speed();
+    ctx->dt_known = false;
+    if (e == hipSuccess && !keep_max) e = launch_clock_reset_max(ctx->clock, ctx->stream);
+    if (e == hipSuccess && !keep_max) e = ctx->cfl_all(ctx->cur);
+    if (e == hipSuccess)
+        e = launch_clock_dt(ctx->clock, clock_fields(ctx, max_cfl, time, max_time, prev_output_time, delta),
+                            &ctx->clock_host->dt, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) return ctx->hip_fail(e, "mh_compute_dt");
-    *dt_out = h.dt;
+    *dt_out = ctx->clock_host->dt;
+    ctx->dt_dev = *dt_out;
+    ctx->dt_known = true;
+    ctx->fold_next = true;
     return MH_OK;
 }
 
@@ -431,11 +455,11 @@ int mh_stage(mh_ctx* ctx, int32_t stage, double dt) {
     if (stage < 0 || stage >= ns) return ctx->fail(MH_ERR_INVALID, "stage out of range for the time stepper");
     if (stage != ctx->next_stage) return ctx->fail(MH_ERR_INVALID, "stages must run in order starting at 0");
     hipError_t e = hipSetDevice(ctx->device);
-    ctx->amax_valid = false;
+    ctx->forget_speed();
     if (stage == 0) ctx->qn = ctx->cur;
     const int in = ctx->cur;
     const int out = (in == ctx->qn) ? (ctx->qn + 1) % 3 : 3 - in - ctx->qn;
-    if (e == hipSuccess) e = launch_clock_set_dt(ctx->clock, dt, ctx->stream);
+    if (e == hipSuccess) e = ctx->set_dt(dt);
     if (e == hipSuccess) e = ctx->stage(in, ctx->qn, out, stage_kind(ctx->sch.stepper, stage), 0);
     ctx->last_in = in;
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
@@ -454,15 +478,17 @@ int mh_time_step(mh_ctx* ctx, double dt) {
     if (!ctx) return MH_ERR_INVALID;
     if (ctx->next_stage != 0) return ctx->fail(MH_ERR_INVALID, "a step is already in progress (mh_stage)");
     hipError_t e = hipSetDevice(ctx->device);
-    ctx->amax_valid = false;
-    if (e == hipSuccess) e = launch_clock_set_dt(ctx->clock, dt, ctx->stream);
+    const bool fold = ctx->fold_next && !ctx->user_fn;
+    ctx->forget_speed();
+    if (e == hipSuccess) e = ctx->set_dt(dt);
     int nc = ctx->cur;
-    if (e == hipSuccess) nc = ctx->enqueue_step(ctx->cur, false, e);
+    if (e == hipSuccess) nc = ctx->enqueue_step(ctx->cur, fold, e);
     if (e == hipSuccess) e = ctx->fill_final(nc);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) return ctx->hip_fail(e, "mh_time_step");
     ctx->cur = nc;
     if (const int rc = tab_check(ctx); rc != MH_OK) return rc;
+    ctx->amax_valid = fold && !ctx->exposed;
     ctx->steps += 1;
     ctx->last_dt = dt;
     return MH_OK;
@@ -477,8 +503,11 @@ int mh_run(mh_ctx* ctx, int64_t nsteps, double max_cfl, double* time, double max
     // speed of the current state in the CFL slots, so only the clock's
     // fields are written; otherwise a CFL pass over the state fills them.
     const bool keep_max = ctx->amax_valid;
-    ctx->amax_valid = false;
-    if (e == hipSuccess) e = write_clock(ctx, max_cfl, *time, max_time, *prev_output_time, delta, keep_max);
+    ctx->forget_speed();
+    ctx->dt_known = false;
+    if (e == hipSuccess)
+        e = launch_clock_start(ctx->clock, clock_fields(ctx, max_cfl, *time, max_time, *prev_output_time, delta),
+                               keep_max ? 0 : 1, ctx->stream);
     if (e == hipSuccess && !keep_max) e = ctx->cfl_all(ctx->cur);
     for (int64_t s = 0; s < nsteps && e == hipSuccess; ++s) {
         const int k = ctx->cur;
@@ -516,10 +545,10 @@ int mh_run(mh_ctx* ctx, int64_t nsteps, double max_cfl, double* time, double max
         ctx->steps += 1;
     }
     if (e == hipSuccess && nsteps > 0) e = ctx->fill_final(ctx->cur);
-    Clock h{};
-    if (e == hipSuccess) e = hipMemcpyAsync(&h, ctx->clock, sizeof(Clock), hipMemcpyDeviceToHost, ctx->stream);
+    if (e == hipSuccess) e = launch_clock_read(ctx->clock, ctx->clock_host, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) return ctx->hip_fail(e, "mh_run");
+    const Clock h = *ctx->clock_host;
     if (const int rc = tab_check(ctx); rc != MH_OK) return rc;
     ctx->amax_valid = true;
     *time = h.time;
@@ -670,7 +699,7 @@ int mh_autotune(mh_ctx* ctx, int32_t steps, const int32_t* candidates, int32_t* 
     }
     ctx->steps = old_steps;
     ctx->cur = start;
-    ctx->amax_valid = false;  // the slots hold a trial state's maximum
+    ctx->forget_speed();  // the slots hold a trial state's maximum
     if (e != hipSuccess) {
         ctx->nspans = old_spans;
         return ctx->hip_fail(e, "mh_autotune");

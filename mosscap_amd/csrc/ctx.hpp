@@ -72,6 +72,7 @@ struct mh_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     int64_t ncells = 0, nvals = 0;
+    std::vector<void*> buffers;  // the device allocations made by mh_create, which the pointers below are into
     double* q64[3] = {nullptr, nullptr, nullptr};
     float* qhi[3] = {nullptr, nullptr, nullptr};
     float* qlo[3] = {nullptr, nullptr, nullptr};
@@ -82,10 +83,33 @@ struct mh_ctx {
     int qn = 0;          // buffer holding Q^n during a step
     int next_stage = 0;  // mh_stage bookkeeping
     // The clock's CFL slots hold the largest signal speed of buffer `cur`
-    // (set by mh_run, whose last stage folds it; cleared by every call that
-    // changes the state or the slots otherwise), so the next mh_run needs no
-    // separate CFL pass.
+    // (set by mh_run and by mh_time_step after mh_compute_dt, whose last stage
+    // folds it; cleared by every call that changes the state or the slots
+    // otherwise), so the next mh_run or mh_compute_dt needs no separate CFL
+    // pass.
     bool amax_valid = false;
+    // mh_compute_dt has just taken a step size and cleared the slots: a caller
+    // that asks for one before each step will ask again, so this step's last
+    // stage folds the maximum
+    bool fold_next = false;
+    // the state's device pointers were given out (mh_device_state outside a
+    // hook): a caller may write it unseen, so mh_compute_dt always rescans
+    bool exposed = false;
+    // step size in the device clock, when the host knows it
+    bool dt_known = false;
+    double dt_dev = 0.0;
+    Clock* clock_host = nullptr;  // pinned: the clock (or its dt) as the last launch wrote it
+    void forget_speed() {
+        amax_valid = false;
+        fold_next = false;
+    }
+    hipError_t set_dt(double dt) {
+        if (dt_known && std::memcmp(&dt, &dt_dev, sizeof(dt)) == 0) return hipSuccess;
+        const hipError_t e = launch_clock_set_dt(clock, dt, stream);
+        dt_known = e == hipSuccess;
+        dt_dev = dt;
+        return e;
+    }
     int nspans = 1;   // spans of the march (march_spans)
     int strips = 0, flat = 0;  // march_columns
     std::string err;
@@ -246,8 +270,7 @@ struct mh_ctx {
         return ghost(src, out, reduce);
     }
 
-    // 2-D and 3-D grids whose faces are all periodic or zerograd, with no
-    // user_bc hook, no tracer fields and no tabulated EOS (its update runs
+    // Grids whose faces are all periodic or zerograd, with no user_bc hook, no tracer fields and no tabulated EOS (its update runs
     // over the ghosts of each stage's input): every ghost is a copy of an
     // interior cell, so the stage kernels read ghost rows, columns and planes
     // from their sources (StageGrid::virt) and a step needs one ghost fill,
@@ -261,8 +284,9 @@ struct mh_ctx {
         const auto copy_bc = [](int32_t b) {
             return b == (int32_t)BoundaryType::Periodic || b == (int32_t)BoundaryType::ZeroGrad;
         };
-        return nd >= 2 && !user_fn && ntr == 0 && !tab_on && copy_bc(bdry.xs) && copy_bc(bdry.xe) &&
-               copy_bc(bdry.ys) && copy_bc(bdry.ye) && (nd < 3 || (copy_bc(bdry.zs) && copy_bc(bdry.ze)));
+        return !user_fn && ntr == 0 && !tab_on && copy_bc(bdry.xs) && copy_bc(bdry.xe) &&
+               (nd < 2 || (copy_bc(bdry.ys) && copy_bc(bdry.ye))) &&
+               (nd < 3 || (copy_bc(bdry.zs) && copy_bc(bdry.ze)));
     }
     void set_virt(StageGrid& g) const {
         g.virt = virtual_ghosts() ? 1 : 0;
@@ -299,7 +323,8 @@ struct mh_ctx {
                 p.gz = grav[2];
                 e = launch_stage3d_f32c(sch, grid3(kind, reduce), p, dz32, stream);
             } else {
-                e = launch_stage1d_f32c(sch, kind, reduce, sz.xc, sz.ng, p, stream);
+                e = launch_stage1d_f32c(sch, kind, reduce, sz.xc, sz.ng, p, stream, virtual_ghosts() ? 1 : 0,
+                                        bdry.xs == (int32_t)BoundaryType::Periodic);
             }
         } else {
             FormF64::Ptrs p{p64(in), p64(qn_k), p64(out), &clock->dt, dx, gamma, amax_slots(clock), nullptr,
@@ -315,7 +340,8 @@ struct mh_ctx {
                 p.gz = grav[2];
                 e = launch_stage3d_f64(sch, grid3(kind, reduce), p, dz64, stream);
             } else {
-                e = launch_stage1d_f64(sch, kind, reduce, sz.xc, sz.ng, p, stream);
+                e = launch_stage1d_f64(sch, kind, reduce, sz.xc, sz.ng, p, stream, virtual_ghosts() ? 1 : 0,
+                                       bdry.xs == (int32_t)BoundaryType::Periodic);
             }
         }
         return e;
@@ -330,8 +356,7 @@ struct mh_ctx {
                         dx, gamma, amax_slots(clock), nullptr, nullptr, nullptr, gravity, grav[0], grav[1]};
         StageGrid g{sz.xc, sz.yc, sz.ng, sz.xc - 2 * sz.ng, sz.yc - 2 * sz.ng, strips, nspans, kind, 0};
         set_virt(g);
-        hipError_t e = nd == 2 ? launch_stage2d_f64(sch, g, p, stream)
-                               : launch_stage1d_f64(sch, kind, 0, sz.xc, sz.ng, p, stream);
+        hipError_t e = launch_stage2d_f64(sch, g, p, stream);  // the adjoint is 2-D
         if (e != hipSuccess || virtual_ghosts()) return e;
         return launch_ghost_f64(nd, ghost_grid(0), FormF64::Planes{(double*)in}, FormF64::Planes{out}, nullptr, stream);
     }
@@ -417,18 +442,16 @@ struct mh_ctx {
         for (int k = 0; k < 3; ++k) {
             if (graph[k]) hipGraphExecDestroy(graph[k]);
             graph[k] = nullptr;
-            if (q64[k]) hipFree(q64[k]);
-            if (qhi[k]) hipFree(qhi[k]);
-            if (qlo[k]) hipFree(qlo[k]);
             q64[k] = nullptr;
             qhi[k] = qlo[k] = nullptr;
         }
         for (hipEvent_t ev : ev_pool) hipEventDestroy(ev);
         ev_pool.clear();
-        for (void* t : {(void*)frx64, (void*)fry64, (void*)wtr64, (void*)frx32, (void*)fry32, (void*)wtr32,
-                        (void*)eos_y, (void*)eos_T, (void*)eos_flag, (void*)dz64, (void*)dz32, (void*)tab_y,
-                        (void*)tab_lT, (void*)tab_yspace, (void*)tab_Tspace, (void*)tab_neg})
+        for (void* t : {(void*)eos_y, (void*)eos_T, (void*)eos_flag, (void*)tab_y, (void*)tab_lT, (void*)tab_yspace,
+                        (void*)tab_Tspace, (void*)tab_neg})
             if (t) hipFree(t);
+        for (void* b : buffers) hipFree(b);
+        buffers.clear();
         tab_y = tab_lT = tab_yspace = tab_Tspace = nullptr;
         tab_neg = nullptr;
         dz64 = nullptr;
@@ -437,9 +460,8 @@ struct mh_ctx {
         frx32 = fry32 = wtr32 = nullptr;
         eos_y = eos_T = nullptr;
         eos_flag = nullptr;
-        if (staging) hipFree(staging);
-        if (clock) hipFree(clock);
-        if (floor_hits) hipFree(floor_hits);
+        if (clock_host) hipHostFree(clock_host);
+        clock_host = nullptr;
         staging = nullptr;
         clock = nullptr;
         floor_hits = nullptr;

@@ -62,19 +62,17 @@ __device__ inline void fold_amax(unsigned long long* slots, uint32_t block, uint
     atomicMax(slots + kAmaxStride * (block & (uint32_t)(kAmaxSlots - 1)), (unsigned long long)m);
 }
 
-// The next step's dt from the CFL slots and the clock (compute_dt_impl's
+// The next step's dt from the CFL slots and the clock's fields (compute_dt_impl's
 // dt_max = dx / max(a), times max_cfl, with the output-time clamp and its
 // nextafter loop, Hydro.cpp:208-240). Called by every lane of one wave (lane
 // l reads slot l); every lane returns the same value. Reads only.
-__device__ inline double clock_next_dt(const Clock* c) {
+__device__ inline double clock_next_dt(const Clock& c, const unsigned long long* slots) {
     static_assert(kAmaxSlots == kWave, "one slot per lane");
-    const unsigned long long* slot =
-        amax_slots(const_cast<Clock*>(c)) + kAmaxStride * (threadIdx.x & (unsigned)(kWave - 1));
-    const double amax = __builtin_bit_cast(double, wave_max_u64(*slot));
-    const double dt_min = c->dx / amax;  // == min over cells of dx / a
-    double dt = dt_min * c->max_cfl;
-    const double t = c->time;
-    const double next_write_time = smin(c->max_time, c->prev_output_time + c->delta);
+    const double amax = __builtin_bit_cast(double, wave_max_u64(slots[kAmaxStride * (threadIdx.x & (unsigned)(kWave - 1))]));
+    const double dt_min = c.dx / amax;  // == min over cells of dx / a
+    double dt = dt_min * c.max_cfl;
+    const double t = c.time;
+    const double next_write_time = smin(c.max_time, c.prev_output_time + c.delta);
     if (t + dt >= next_write_time) {
         dt = next_write_time - t;
         while (t + dt < next_write_time) {
@@ -82,6 +80,9 @@ __device__ inline double clock_next_dt(const Clock* c) {
         }
     }
     return dt;
+}
+__device__ inline double clock_next_dt(const Clock* c) {
+    return clock_next_dt(*c, amax_slots(const_cast<Clock*>(c)));
 }
 
 // time += dt and, once an output time is reached, prev_output_time = time

@@ -184,6 +184,28 @@ __global__ void clock_reset_max_kernel(Clock* c) {
     if (blockIdx.x == 0 && threadIdx.x < kAmaxSlots) amax_slots(c)[kAmaxStride * threadIdx.x] = 0ull;
 }
 
+// The clock's fields from the launch's arguments: no copy from host memory.
+// With `reset` the CFL slots are cleared.
+__global__ void clock_start_kernel(Clock* c, Clock fields, int reset) {
+    if (threadIdx.x == 0) *c = fields;
+    if (reset) amax_slots(c)[kAmaxStride * threadIdx.x] = 0ull;
+}
+
+// A host loop's compute_dt in one launch: the clock's fields from the
+// arguments, dt from the CFL slots, which are cleared for the next step's
+// fold, and dt again into the caller's pinned host memory (no copy back).
+__global__ void clock_dt_kernel(Clock* c, Clock fields, double* host_dt) {
+    fields.dt = clock_next_dt(fields, amax_slots(c));
+    amax_slots(c)[kAmaxStride * threadIdx.x] = 0ull;  // after every lane has read its slot (wave order)
+    if (threadIdx.x != 0) return;
+    *c = fields;
+    *host_dt = fields.dt;
+}
+
+__global__ void clock_read_kernel(const Clock* c, Clock* host) {
+    if (threadIdx.x == 0) *host = *c;
+}
+
 }  // namespace
 
 hipError_t launch_ghost_f64(int nd, const GhostGrid& g, FormF64::Planes in, FormF64::Planes out,
@@ -286,6 +308,19 @@ hipError_t launch_clock_set_dt(Clock* c, double dt, hipStream_t st) {
 }
 hipError_t launch_clock_reset_max(Clock* c, hipStream_t st) {
     hipLaunchKernelGGL(clock_reset_max_kernel, dim3(1), dim3(64), 0, st, c);
+    return hipGetLastError();
+}
+
+hipError_t launch_clock_start(Clock* c, const Clock& fields, int reset, hipStream_t st) {
+    hipLaunchKernelGGL(clock_start_kernel, dim3(1), dim3(kWave), 0, st, c, fields, reset);
+    return hipGetLastError();
+}
+hipError_t launch_clock_dt(Clock* c, const Clock& fields, double* host_dt, hipStream_t st) {
+    hipLaunchKernelGGL(clock_dt_kernel, dim3(1), dim3(kWave), 0, st, c, fields, host_dt);
+    return hipGetLastError();
+}
+hipError_t launch_clock_read(const Clock* c, Clock* host, hipStream_t st) {
+    hipLaunchKernelGGL(clock_read_kernel, dim3(1), dim3(kWave), 0, st, c, host);
     return hipGetLastError();
 }
 

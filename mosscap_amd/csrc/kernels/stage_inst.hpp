@@ -32,6 +32,7 @@ void stage2d_kernel(StageGrid g, typename Form::Ptrs p) {
 
 struct Stage1dGrid {
     int32_t xc, ng, nx, kind, reduce_dt;
+    int32_t virt, per;  // ghosts read from their sources (StageGrid::virt; periodic `per`, else zerograd)
 };
 
 template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS>
@@ -44,7 +45,8 @@ __global__ __launch_bounds__(64) void stage1d_kernel(Stage1dGrid g, typename For
     const T dtdx = dt / (T)p.dx;
     double amax = 0.0;
     unsigned int hits = 0;
-    stage1d_segment<Form, R, SL, RS>(p, g.kind, g.reduce_dt, 0, g.xc, g.ng, g.nx, i0, dtdx, dt, lds, amax, hits);
+    stage1d_segment<Form, R, SL, RS>(p, g.kind, g.reduce_dt, 0, g.xc, g.ng, g.nx, i0, dtdx, dt, lds, amax, hits,
+                                     Form::kVirtualGhosts ? g.virt : 0, g.per != 0);
     if (g.reduce_dt) {
         const uint64_t m = wave_max_u64(__builtin_bit_cast(uint64_t, amax));
         if (threadIdx.x == 0) atomicMax(p.amax_bits, (unsigned long long)m);
@@ -127,12 +129,12 @@ hipError_t launch_stage2d_impl(const Schemes& s, const StageGrid& g, const typen
 
 template <class Form>
 hipError_t launch_stage1d_impl(const Schemes& s, int kind, int reduce_dt, int xc, int ng,
-                               const typename Form::Ptrs& p, hipStream_t st) {
+                               const typename Form::Ptrs& p, hipStream_t st, int virt, int per) {
     const int nx = xc - 2 * ng;
     if (nx < 1 || ng < min_ghost_cells(s.recon)) return hipErrorInvalidValue;
     auto pick = [&]<Reconstruction R, SlopeLimiter SL>() { return SolverPick<Form, R, SL>::one(s.solver); };
     Stage1dFn<Form> fn = pick_scheme<Form>(s, pick);
-    const Stage1dGrid g{xc, ng, nx, kind, reduce_dt};
+    const Stage1dGrid g{xc, ng, nx, kind, reduce_dt, virt, per};
     const int segs = (nx + kStripOut - 1) / kStripOut;
     hipLaunchKernelGGL(fn, dim3((unsigned)segs), dim3(kWave), 0, st, g, p);
     return hipGetLastError();

@@ -70,11 +70,12 @@ hipError_t launch_stage3d_f64(const Schemes& s, const StageGrid& g, const FormF6
                               hipStream_t st);
 hipError_t launch_stage3d_f32c(const Schemes& s, const StageGrid& g, const FormF32c::Ptrs& p, float* dz,
                                hipStream_t st);
-// 1-D stage over one row of xc cells (ng ghosts each side).
+// 1-D stage over one row of xc cells (ng ghosts each side); virt: ghosts read
+// from their sources, per: periodic, else zerograd.
 hipError_t launch_stage1d_f64(const Schemes& s, int kind, int reduce_dt, int xc, int ng, const FormF64::Ptrs& p,
-                              hipStream_t st);
+                              hipStream_t st, int virt = 0, int per = 0);
 hipError_t launch_stage1d_f32c(const Schemes& s, int kind, int reduce_dt, int xc, int ng, const FormF32c::Ptrs& p,
-                               hipStream_t st);
+                               hipStream_t st, int virt = 0, int per = 0);
 
 // Tracer planes of a 2-D stage (p.frx / p.fry hold the stage's density fluxes).
 hipError_t launch_tracer_f64(const Schemes& s, const TracerGrid& g, const FormF64::Ptrs& p, double* wtr,
@@ -117,6 +118,12 @@ hipError_t launch_tab_eos_f32c(int nd, FormF32c::Planes in, FormF32c::Planes out
 hipError_t launch_clock_finalize(Clock* c, int advance, hipStream_t st);
 hipError_t launch_clock_set_dt(Clock* c, double dt, hipStream_t st);
 hipError_t launch_clock_reset_max(Clock* c, hipStream_t st);
+// The clock's fields from the host (and its CFL slots cleared, with reset);
+// those and the step size they and the slots give, also into pinned host
+// memory; the clock into pinned host memory.
+hipError_t launch_clock_start(Clock* c, const Clock& fields, int reset, hipStream_t st);
+hipError_t launch_clock_dt(Clock* c, const Clock& fields, double* host_dt, hipStream_t st);
+hipError_t launch_clock_read(const Clock* c, Clock* host, hipStream_t st);
 
 // Conversions between the FP64 layout and the compensated hi/lo planes.
 hipError_t launch_split_f64_to_f32c(const double* src, FormF32c::Planes dst, int n, hipStream_t st);
