@@ -107,8 +107,9 @@ struct Arith<Dual<N>> {
 // cons_to_prim (Eos.hpp:61-79), 2-D: w = (rho, mx/rho, my/rho, (g-1)(E - (rho/2)|v|^2)).
 __host__ __device__ inline void cons_to_prim_vjp2(double gamma, const double (&q)[4], const double (&lw)[4],
                                                   double (&lq)[4]) {
+#pragma clang fp contract(fast)
     const double rho = q[0];
-    const double ir = 1.0 / rho;
+    const double ir = Recip<double>(rho).mul(1.0);
     const double vx = q[1] * ir, vy = q[2] * ir;
     const double gm1 = gamma - 1.0;
     lq[0] = lw[0] - (vx * lw[1] + vy * lw[2]) * ir + gm1 * 0.5 * (vx * vx + vy * vy) * lw[3];
@@ -119,29 +120,46 @@ __host__ __device__ inline void cons_to_prim_vjp2(double gamma, const double (&q
 
 // WENO5-Z (Reconstruct.hpp:217-274): given the cotangents lL, lR of the
 // left/right face values of the cell, accumulate d(lL*wL + lR*wR)/ds into ls.
-__host__ __device__ inline void weno5z_vjp(const double (&s)[5], double lL, double lR, double (&ls)[5]) {
+// What decides a branch (the sign of beta0 - beta2) is computed as the forward
+// does; the rest multiplies by the five reciprocals of the cell's denominators
+// (12 divisions otherwise) and fuses its multiply-adds.
+struct WenoParts {
+    double a[3], b[3], be[3];
+};
+__host__ __device__ inline WenoParts weno5z_parts(const double (&s)[5]) {
     const double sm2 = s[0], sm1 = s[1], s0 = s[2], sp1 = s[3], sp2 = s[4];
-    const double c0 = 13.0 / 12.0, c1 = 0.25, eps = 1e-36;
+    const double c0 = 13.0 / 12.0, c1 = 0.25;
     const double a0 = sm2 - 2.0 * sm1 + s0, b0 = sm2 - 4.0 * sm1 + 3.0 * s0;
     const double a1 = sm1 - 2.0 * s0 + sp1, b1 = sm1 - sp1;
     const double a2 = s0 - 2.0 * sp1 + sp2, b2 = 3.0 * s0 - 4.0 * sp1 + sp2;
-    const double be[3] = {c0 * a0 * a0 + c1 * b0 * b0, c0 * a1 * a1 + c1 * b1 * b1, c0 * a2 * a2 + c1 * b2 * b2};
+    return {{a0, a1, a2},
+            {b0, b1, b2},
+            {c0 * a0 * a0 + c1 * b0 * b0, c0 * a1 * a1 + c1 * b1 * b1, c0 * a2 * a2 + c1 * b2 * b2}};
+}
+__host__ __device__ inline void weno5z_vjp(const double (&s)[5], double lL, double lR, double (&ls)[5]) {
+#pragma clang fp contract(fast)
+    const double sm2 = s[0], sm1 = s[1], s0 = s[2], sp1 = s[3], sp2 = s[4];
+    const double c0 = 13.0 / 12.0, c1 = 0.25, eps = 1e-36;
+    const WenoParts w = weno5z_parts(s);
+    const double(&be)[3] = w.be;
     const double dtau = be[0] - be[2];
     const double tau = __builtin_fabs(dtau);
+    const Recip<double> r[3] = {Recip<double>(be[0] + eps), Recip<double>(be[1] + eps), Recip<double>(be[2] + eps)};
     double ind[3], q[3];
     for (int k = 0; k < 3; ++k) {
-        ind[k] = tau / (be[k] + eps);
+        ind[k] = r[k].mul(tau);
         q[k] = 1.0 + ind[k] * ind[k];
     }
     const double eL[3] = {2.0 * s0 + 5.0 * sm1 - sm2, -sp1 + 5.0 * s0 + 2.0 * sm1, 2.0 * sp2 - 7.0 * sp1 + 11.0 * s0};
     const double eR[3] = {2.0 * s0 + 5.0 * sp1 - sp2, -sm1 + 5.0 * s0 + 2.0 * sp1, 2.0 * sm2 - 7.0 * sm1 + 11.0 * s0};
     const double aL[3] = {3.0 * q[0], 6.0 * q[1], q[2]};
     const double aR[3] = {3.0 * q[2], 6.0 * q[1], q[0]};
-    const double NL = eL[0] * aL[0] + eL[1] * aL[1] + eL[2] * aL[2], DL = 6.0 * (aL[0] + aL[1] + aL[2]);
-    const double NR = eR[0] * aR[0] + eR[1] * aR[1] + eR[2] * aR[2], DR = 6.0 * (aR[0] + aR[1] + aR[2]);
+    const double NL = eL[0] * aL[0] + eL[1] * aL[1] + eL[2] * aL[2];
+    const double NR = eR[0] * aR[0] + eR[1] * aR[1] + eR[2] * aR[2];
+    const Recip<double> DL(6.0 * (aL[0] + aL[1] + aL[2])), DR(6.0 * (aR[0] + aR[1] + aR[2]));
     // wL = NL/DL, wR = NR/DR
-    const double lNL = lL / DL, lDL = -lL * (NL / DL) / DL;
-    const double lNR = lR / DR, lDR = -lR * (NR / DR) / DR;
+    const double lNL = DL.mul(lL), lDL = -lNL * DL.mul(NL);
+    const double lNR = DR.mul(lR), lDR = -lNR * DR.mul(NR);
     double laL[3], laR[3], leL[3], leR[3];
     for (int k = 0; k < 3; ++k) {
         laL[k] = lNL * eL[k] + 6.0 * lDL;
@@ -155,17 +173,16 @@ __host__ __device__ inline void weno5z_vjp(const double (&s)[5], double lL, doub
     lq[2] = laL[2] + 3.0 * laR[0];
     double ltau = 0.0, lbe[3];
     for (int k = 0; k < 3; ++k) {
-        const double lind = 2.0 * ind[k] * lq[k];
-        const double r = 1.0 / (be[k] + eps);
-        ltau += lind * r;
-        lbe[k] = -lind * ind[k] * r;
+        const double lr = r[k].mul(2.0 * ind[k] * lq[k]);
+        ltau += lr;
+        lbe[k] = -lr * ind[k];
     }
     const double sg = dtau > 0.0 ? 1.0 : (dtau < 0.0 ? -1.0 : 0.0);
     lbe[0] += sg * ltau;
     lbe[2] -= sg * ltau;
-    const double la0 = 2.0 * c0 * a0 * lbe[0], lb0 = 2.0 * c1 * b0 * lbe[0];
-    const double la1 = 2.0 * c0 * a1 * lbe[1], lb1 = 2.0 * c1 * b1 * lbe[1];
-    const double la2 = 2.0 * c0 * a2 * lbe[2], lb2 = 2.0 * c1 * b2 * lbe[2];
+    const double la0 = 2.0 * c0 * w.a[0] * lbe[0], lb0 = 2.0 * c1 * w.b[0] * lbe[0];
+    const double la1 = 2.0 * c0 * w.a[1] * lbe[1], lb1 = 2.0 * c1 * w.b[1] * lbe[1];
+    const double la2 = 2.0 * c0 * w.a[2] * lbe[2], lb2 = 2.0 * c1 * w.b[2] * lbe[2];
     // stencil coefficients of a, b and the ENO candidates over (s-2, s-1, s0, s1, s2)
     ls[0] += la0 + lb0 - leL[0] + 2.0 * leR[2];
     ls[1] += -2.0 * la0 - 4.0 * lb0 + la1 + lb1 + 5.0 * leL[0] + 2.0 * leL[1] - leR[1] - 7.0 * leR[2];
@@ -179,18 +196,19 @@ __host__ __device__ inline void weno5z_vjp(const double (&s)[5], double lL, doub
 template <int Axis>
 __host__ __device__ inline void rusanov_vjp2(double gamma, const double (&wL)[4], const double (&wR)[4],
                                              const double (&lf)[4], double (&lwL)[4], double (&lwR)[4]) {
+#pragma clang fp contract(fast)
     constexpr int IV = 1 + Axis;
-    const double gm1 = gamma - 1.0;
+    const Recip<double> igm1(gamma - 1.0);
     auto side = [&](const double (&w)[4], double sgn_q, double (&lw)[4], double& cs_out, double (&q)[4]) {
         const double rho = w[0], vx = w[1], vy = w[2], p = w[3];
         const double vn = w[IV];
         const double v2 = vx * vx + vy * vy;
-        const double E = p / gm1 + 0.5 * rho * v2;
+        const double E = igm1.div(p) + 0.5 * rho * v2;
         q[0] = rho;
         q[1] = rho * vx;
         q[2] = rho * vy;
         q[3] = E;
-        cs_out = __builtin_sqrt(gamma * p / rho);
+        cs_out = Arith<double>::sqrt_mid(Arith<double>::div(gamma * p, rho));
         const double H = E + p;
         // 0.5 * J_f^T lf
         double g[4];
@@ -199,7 +217,7 @@ __host__ __device__ inline void rusanov_vjp2(double gamma, const double (&wL)[4]
                       (Axis == 0 ? rho * vy : 0.0) * lf[2] + (rho * vx * vn + (Axis == 0 ? H : 0.0)) * lf[3]);
         g[2] = 0.5 * ((Axis == 1 ? rho : 0.0) * lf[0] + (Axis == 1 ? rho * vx : 0.0) * lf[1] +
                       (rho * vn + (Axis == 1 ? rho * vy : 0.0)) * lf[2] + (rho * vy * vn + (Axis == 1 ? H : 0.0)) * lf[3]);
-        g[3] = 0.5 * ((Axis == 0 ? 1.0 : 0.0) * lf[1] + (Axis == 1 ? 1.0 : 0.0) * lf[2] + (1.0 / gm1 + 1.0) * vn * lf[3]);
+        g[3] = 0.5 * ((Axis == 0 ? 1.0 : 0.0) * lf[1] + (Axis == 1 ? 1.0 : 0.0) * lf[2] + (igm1.mul(1.0) + 1.0) * vn * lf[3]);
         // -/+ 0.5 * max_c * J_q^T lf (sgn_q = +1 on the left, -1 on the right)
         // (stored for the caller to scale by max_c)
         lw[0] = g[0];
@@ -218,7 +236,7 @@ __host__ __device__ inline void rusanov_vjp2(double gamma, const double (&wL)[4]
         o[0] = lf[0] + vx * lf[1] + vy * lf[2] + 0.5 * (vx * vx + vy * vy) * lf[3];
         o[1] = rho * lf[1] + rho * vx * lf[3];
         o[2] = rho * lf[2] + rho * vy * lf[3];
-        o[3] = lf[3] / gm1;
+        o[3] = igm1.mul(lf[3]);
     };
     double jqL[4], jqR[4];
     jq(wL, jqL);
@@ -230,8 +248,10 @@ __host__ __device__ inline void rusanov_vjp2(double gamma, const double (&wL)[4]
     auto dcs = [&](const double (&w)[4], double cs, double (&o)[4]) {
         // cs = sqrt(g p / rho): dcs/drho = -cs/(2 rho), dcs/dp = g / (2 rho cs)
         const double lcs = 0.5 * lc;
-        o[0] += lcs * (-cs / (2.0 * w[0]));
-        o[3] += lcs * (gamma / (2.0 * w[0] * cs));
+        // = cs / (2p)
+        const double h = 0.5 * lcs * cs;
+        o[0] -= Recip<double>(w[0]).mul(h);
+        o[3] += Recip<double>(w[3]).mul(h);
         const double vn = w[IV];
         const double sg = vn > 0.0 ? 1.0 : (vn < 0.0 ? -1.0 : 0.0);
         o[IV] += lcs * sg;
@@ -245,7 +265,8 @@ __host__ __device__ inline void rusanov_vjp2(double gamma, const double (&wL)[4]
 }
 
 // HLLC (Riemann.hpp:75-176), 2-D along Axis: the forward sequence of
-// riemann_flux<Hllc> replayed, then its reverse sweep; J^T lf accumulated into
+// riemann_flux<Hllc> replayed (the same operations, so the same branches), then
+// its reverse sweep through the forward's reciprocals; J^T lf accumulated into
 // lwL, lwR. Branches (wave-speed switches, the floors on bM/bP and cp) pass the
 // derivative of the branch the forward values took.
 template <int Axis>
@@ -257,21 +278,23 @@ __host__ __device__ inline void hllc_vjp2(double gamma, const double (&wL)[4], c
     const double rL = wL[0], rR = wR[0], pL = wL[3], pR = wR[3];
     const double uL = wL[IV], uR = wR[IV];
     // ---- forward (same operations as the functor) ----
-    const double csL = __builtin_sqrt(gamma * pL / rL);
-    const double csR = __builtin_sqrt(gamma * pR / rR);
+    using A = Arith<double>;
+    const Recip<double> irL(rL), irR(rR), ipL(pL), ipR(pR), igm1(gm1);
+    const double csL = A::sqrt_mid(A::div(gamma * pL, rL));
+    const double csR = A::sqrt_mid(A::div(gamma * pR, rR));
     const double v2L = wL[1] * wL[1] + wL[2] * wL[2];
     const double v2R = wR[1] * wR[1] + wR[2] * wR[2];
     const double qLm = rL * uL, qRm = rR * uR;
-    const double qLe = pL / gm1 + 0.5 * rL * v2L;
-    const double qRe = pR / gm1 + 0.5 * rR * v2R;
+    const double qLe = igm1.div(pL) + 0.5 * rL * v2L;
+    const double qRe = igm1.div(pR) + 0.5 * rR * v2R;
     const double rho_avg = 0.5 * (rL + rR);
     const double cs_avg = 0.5 * (csL + csR);
     const double K = uL - uR;
     const double p_mid = 0.5 * (pL + pR + K * rho_avg * cs_avg);
-    const double g_fac = (gamma + 1.0) / (2.0 * gamma);
+    const double g_fac = A::div(gamma + 1.0, 2.0 * gamma);
     const bool lo_L = p_mid <= pL, lo_R = p_mid <= pR;
-    const double cLs = lo_L ? 1.0 : __builtin_sqrt(1.0 + g_fac * (p_mid / pL - 1.0));
-    const double cRs = lo_R ? 1.0 : __builtin_sqrt(1.0 + g_fac * (p_mid / pR - 1.0));
+    const double cLs = lo_L ? 1.0 : A::sqrt_mid(1.0 + g_fac * (A::div(p_mid, pL) - 1.0));
+    const double cRs = lo_R ? 1.0 : A::sqrt_mid(1.0 + g_fac * (A::div(p_mid, pR) - 1.0));
     const double aL = uL - csL * cLs;
     const double aR = uR + csR * cRs;
     const bool bM_is_aL = aL < -tiny, bP_is_aR = tiny < aR;
@@ -280,9 +303,9 @@ __host__ __device__ inline void hllc_vjp2(double gamma, const double (&wL)[4], c
     const double vL1 = uL - aL, vR1 = uR - aR;
     const double tL = pL + vL1 * qLm, tR = pR + vR1 * qRm;
     const double mL = rL * vL1, mR = -(rR * vR1);
-    const double inv_m = mL + mR;
-    const double aM = (tL - tR) / inv_m;
-    const double cp0 = (mL * tR + mR * tL) / inv_m;
+    const Recip<double> inv_m(mL + mR);
+    const double aM = inv_m.div(tL - tR);
+    const double cp0 = inv_m.div(mL * tR + mR * tL);
     const bool cp_pass = !(cp0 < 0.0);
     const double cp = cp_pass ? cp0 : 0.0;
     const double vL2 = uL - bM, vR2 = uR - bP;
@@ -292,11 +315,14 @@ __host__ __device__ inline void hllc_vjp2(double gamma, const double (&wL)[4], c
     fL[IV] += pL;
     fR[IV] += pR;
     const bool pos = aM >= 0.0;
-    const double d = pos ? aM - bM : bP - aM;
-    const double sL = pos ? aM / d : 0.0;
-    const double sR = pos ? 0.0 : -aM / d;
-    const double sM = pos ? -bM / d : bP / d;
-    // ---- reverse ----
+    const Recip<double> d(pos ? aM - bM : bP - aM);
+    const double sK = d.div(pos ? aM : -aM);
+    const double sL = pos ? sK : 0.0;
+    const double sR = pos ? 0.0 : sK;
+    const double sM = d.div(pos ? -bM : bP);
+    // ---- reverse (its multiply-adds fused) ----
+    {
+#pragma clang fp contract(fast)
     double gL[4] = {0.0, 0.0, 0.0, 0.0}, gR[4] = {0.0, 0.0, 0.0, 0.0};  // cotangents of wL, wR
     const double smcp = sM * cp;
     double l_sL = 0.0, l_sR = 0.0;
@@ -310,13 +336,13 @@ __host__ __device__ inline void hllc_vjp2(double gamma, const double (&wL)[4], c
     double l_aM = lf[3] * smcp;
     double l_bM = 0.0, l_bP = 0.0;
     if (pos) {
-        const double l_d = -(l_sL * sL + l_sM * sM) / d;
-        l_aM += l_sL / d + l_d;
-        l_bM += -l_sM / d - l_d;
+        const double l_d = -d.mul(l_sL * sL + l_sM * sM);
+        l_aM += d.mul(l_sL) + l_d;
+        l_bM += -d.mul(l_sM) - l_d;
     } else {
-        const double l_d = -(l_sR * sR + l_sM * sM) / d;
-        l_aM += -l_sR / d - l_d;
-        l_bP += l_sM / d + l_d;
+        const double l_d = -d.mul(l_sR * sR + l_sM * sM);
+        l_aM += -d.mul(l_sR) - l_d;
+        l_bP += d.mul(l_sM) + l_d;
     }
     // fL, fR
     auto side_f = [&](const double (&w)[4], double s, double mf, double v2, double qe, double p, double u,
@@ -344,16 +370,17 @@ __host__ __device__ inline void hllc_vjp2(double gamma, const double (&wL)[4], c
     // cp = max(cp0, 0); cp0 = (mL*tR + mR*tL) / inv_m; aM = (tL - tR) / inv_m
     double l_mL = 0.0, l_mR = 0.0, l_tL = 0.0, l_tR = 0.0, l_inv = 0.0;
     if (cp_pass) {
-        const double l_n = l_cp / inv_m;
-        l_inv -= l_cp * cp0 / inv_m;
+        const double l_n = inv_m.mul(l_cp);
+        l_inv -= l_n * cp0;
         l_mL += l_n * tR;
         l_tR += l_n * mL;
         l_mR += l_n * tL;
         l_tL += l_n * mR;
     }
-    l_tL += l_aM / inv_m;
-    l_tR -= l_aM / inv_m;
-    l_inv -= l_aM * aM / inv_m;
+    const double l_a = inv_m.mul(l_aM);
+    l_tL += l_a;
+    l_tR -= l_a;
+    l_inv -= l_a * aM;
     l_mL += l_inv;
     l_mR += l_inv;
     // mR = -(rR*vR1), mL = rL*vL1, tX = pX + vX1*qXm
@@ -378,14 +405,14 @@ __host__ __device__ inline void hllc_vjp2(double gamma, const double (&wL)[4], c
     const double l_cRs = l_aR * csR, l_cLs = -l_aL * csL;
     double l_pmid = 0.0;
     if (!lo_R) {
-        const double l_x = l_cRs / (2.0 * cRs) * g_fac;  // d/d(p_mid/pR)
-        l_pmid += l_x / pR;
-        gR[3] -= l_x * (p_mid / pR) / pR;
+        const double l_x = ipR.mul(l_cRs / (2.0 * cRs) * g_fac);  // d/d(p_mid/pR), over pR
+        l_pmid += l_x;
+        gR[3] -= l_x * ipR.mul(p_mid);
     }
     if (!lo_L) {
-        const double l_x = l_cLs / (2.0 * cLs) * g_fac;
-        l_pmid += l_x / pL;
-        gL[3] -= l_x * (p_mid / pL) / pL;
+        const double l_x = ipL.mul(l_cLs / (2.0 * cLs) * g_fac);
+        l_pmid += l_x;
+        gL[3] -= l_x * ipL.mul(p_mid);
     }
     // p_mid = 0.5*(pL + pR + (K*rho_avg)*cs_avg)
     const double l_h = 0.5 * l_pmid;
@@ -403,22 +430,24 @@ __host__ __device__ inline void hllc_vjp2(double gamma, const double (&wL)[4], c
     // q: qXm = rX*uX, qXe = pX/gm1 + 0.5*rX*|v|^2
     gL[0] += l_qLm * uL + l_qLe * 0.5 * v2L;
     gL[IV] += l_qLm * rL;
-    gL[3] += l_qLe / gm1;
+    gL[3] += igm1.mul(l_qLe);
     gL[1] += l_qLe * rL * wL[1];
     gL[2] += l_qLe * rL * wL[2];
     gR[0] += l_qRm * uR + l_qRe * 0.5 * v2R;
     gR[IV] += l_qRm * rR;
-    gR[3] += l_qRe / gm1;
+    gR[3] += igm1.mul(l_qRe);
     gR[1] += l_qRe * rR * wR[1];
     gR[2] += l_qRe * rR * wR[2];
-    // cs = sqrt(gamma*p/rho)
-    gL[3] += l_csL * gamma / (2.0 * rL * csL);
-    gL[0] -= l_csL * csL / (2.0 * rL);
-    gR[3] += l_csR * gamma / (2.0 * rR * csR);
-    gR[0] -= l_csR * csR / (2.0 * rR);
+    // cs = sqrt(gamma*p/rho): dcs/dp = cs/(2p), dcs/drho = -cs/(2rho)
+    const double hL = 0.5 * l_csL * csL, hR = 0.5 * l_csR * csR;
+    gL[3] += ipL.mul(hL);
+    gL[0] -= irL.mul(hL);
+    gR[3] += ipR.mul(hR);
+    gR[0] -= irR.mul(hR);
     for (int k = 0; k < 4; ++k) {
         lwL[k] += gL[k];
         lwR[k] += gR[k];
+    }
     }
 }
 

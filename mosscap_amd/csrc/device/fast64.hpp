@@ -77,6 +77,7 @@ struct Recip {
     T b;
     __host__ __device__ explicit Recip(const T& x) : b(x) {}
     __host__ __device__ T div(const T& a) const { return a / b; }
+    __host__ __device__ T mul(const T& a) const { return a / b; }
 };
 template <>
 struct Recip<double> {
@@ -88,9 +89,11 @@ struct Recip<double> {
         const double q = a * r;
         return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), r, q), b, a);
     }
+    __device__ double mul(double a) const { return a * r; }  // a / b to an ulp
 #else
     __host__ __device__ explicit Recip(double x) : b(x) {}
     __host__ __device__ double div(double a) const { return a / b; }
+    __host__ __device__ double mul(double a) const { return a / b; }
 #endif
 };
 
