@@ -43,7 +43,7 @@ struct LineArgs {
     double* acc;
     double a_qn, a_qs, a_l;
     int32_t acc_mode;  // AdjStage::acc_mode
-    int32_t nseg;
+    int32_t nseg, nlines;  // segments per line, lines
     // the axis is periodic on both faces: its lines are circular (positions
     // run over the interior, halo positions wrap), so no contribution lands
     // in a ghost cell and that axis needs no transposed ghost fill
@@ -62,6 +62,16 @@ __device__ inline void face_vjp(double gamma, const double (&wl)[4], const doubl
     }
 }
 
+// Lines per workgroup, one wavefront each. In the x sweep a line is a row and
+// a wavefront's lanes read neighbouring cells. In the y sweep a line is a
+// column: a wavefront alone reads 64 cache lines for 64 cells, so four
+// neighbouring columns are loaded, and their results stored, by the four
+// wavefronts together, 16 rows of four cells per instruction (512^2: 37 us a
+// sweep with a column per workgroup, 29 us so; three such workgroups fit a CU,
+// one of eight columns would leave a third of its wavefronts out).
+template <int Axis>
+constexpr int kLines = Axis == 0 ? 1 : 4;
+
 // One wavefront per (line, segment). Axis 0: lines are the interior rows,
 // positions run over all columns (over the interior columns, wrapping, when x
 // is circular). Axis 1: lines are all columns (ghost columns only carry the x
@@ -69,38 +79,49 @@ __device__ inline void face_vjp(double gamma, const double (&wl)[4], const doubl
 // circular), positions run over all rows (the interior rows, wrapping, when
 // y is circular).
 template <Reconstruction R, SlopeLimiter SL, RiemannSolver RS, int Axis>
-__global__ __launch_bounds__(64) void adj_line_kernel(LineArgs a) {
+__global__ __launch_bounds__(kWave * kLines<Axis>) void adj_line_kernel(LineArgs a) {
     constexpr int ORD = stencil_order(R);
     constexpr int HALO = 2 * ORD + 1;
     constexpr int OUT = kWave - 2 * HALO;
-    // 8 KB of LDS per wave, so that 4 waves fit each SIMD
-    __shared__ double sW[4][kWave], sWR[4][kWave], sMu[4][kWave], sLR[4][kWave];
+    constexpr int L = kLines<Axis>;
+    // 8 KB of LDS per wave, so that 4 waves fit each SIMD; the pad puts the
+    // lines' words on different banks
+    struct Lds {
+        double W[4][kWave], WR[4][kWave], Mu[4][kWave], LR[4][kWave], pad[L > 1 ? 4 : 1];
+    };
+    __shared__ Lds lds[L];
+    const auto sync = [] {
+        if constexpr (L > 1) __syncthreads();
+        else wave_lds_sync();
+    };
 
     const AdjGrid& g = a.g;
-    const int t = threadIdx.x;
     // Logical block ids run contiguously within each XCD (xcd_remap), so
     // neighbouring lines share an L2. The x sweep keeps a row's segments
     // adjacent (they share halo cells); the y sweep takes columns fastest, so
-    // the 16 neighbouring columns that share each cache line of a row run
-    // together.
+    // the columns that share each cache line of a row run together.
     const uint32_t lb = xcd_remap(blockIdx.x, gridDim.x);
-    const uint32_t nlines = gridDim.x / (uint32_t)a.nseg;
-    const int seg = Axis == 0 ? (int)(lb % (uint32_t)a.nseg) : (int)(lb / nlines);
-    const int line = Axis == 0 ? (int)(lb / (uint32_t)a.nseg) : (int)(lb % nlines);
+    const uint32_t ngroups = gridDim.x / (uint32_t)a.nseg;
+    const int seg = Axis == 0 ? (int)(lb % (uint32_t)a.nseg) : (int)(lb / ngroups);
+    const int line0 = (Axis == 0 ? (int)(lb / (uint32_t)a.nseg) : (int)(lb % ngroups)) * L;
     const int len = Axis == 0 ? g.xc : g.yc;
     const int nax = Axis == 0 ? g.nx : g.ny;
     const bool circ = (Axis == 0 ? a.circ_x : a.circ_y) != 0;
-    // position along the line (with ghosts); circular lines number the
-    // interior from 0 and read a position outside it at its periodic image
-    const int p = circ ? g.ng + seg * OUT - HALO + t : seg * OUT - HALO + t;
-    const int pc = circ ? g.ng + ((p - g.ng) % nax + nax) % nax : min(max(p, 0), len - 1);
-    const int li = Axis == 0 ? g.ng + line : (a.circ_x ? g.ng + line : line);  // row (axis 0) or column (axis 1)
-    const bool line_in = Axis == 0 ? true : (li >= g.ng && li < g.ng + g.nx);
-    const int cell = Axis == 0 ? li * g.xc + pc : pc * g.xc + li;
-    const int i = Axis == 0 ? pc : li, j = Axis == 0 ? li : pc;
-    const bool cell_in = i >= g.ng && i < g.ng + g.nx && j >= g.ng && j < g.ng + g.ny;
     const int nc = g.ncells;
+    // position `at` of the segment along its line (with ghosts); circular lines
+    // number the interior from 0 and read a position outside it at its periodic
+    // image
+    auto position = [&](int at) { return circ ? g.ng + seg * OUT - HALO + at : seg * OUT - HALO + at; };
+    auto line_index = [&](int line) { return Axis == 0 ? g.ng + line : (a.circ_x ? g.ng + line : line); };
 
+    // ---- the cell this thread loads and, at the end, stores ----------------
+    const int lt = (int)threadIdx.x / L, lc = (int)threadIdx.x % L;  // position and line of the group
+    const int lp = position(lt);
+    const int pc = circ ? g.ng + ((lp - g.ng) % nax + nax) % nax : min(max(lp, 0), len - 1);
+    const int ll = line_index(min(line0 + lc, a.nlines - 1));  // row (axis 0) or column (axis 1)
+    const int i = Axis == 0 ? pc : ll, j = Axis == 0 ? ll : pc;
+    const int cell = j * g.xc + i;
+    const bool cell_in = i >= g.ng && i < g.ng + g.nx && j >= g.ng && j < g.ng + g.ny;
     const int qcell = g.virt ? copy_ghost_source(j, g.ny, g.ng, g.yper) * g.xc + copy_ghost_source(i, g.nx, g.ng, g.xper)
                              : cell;
     double qq[4], mu[4];
@@ -114,12 +135,19 @@ __global__ __launch_bounds__(64) void adj_line_kernel(LineArgs a) {
         cons_to_prim<2>(g.gamma, qq, w);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            sW[v][t] = w[v];
-            sMu[v][t] = mu[v];
-            sLR[v][t] = 0.0;
+            lds[lc].W[v][lt] = w[v];
+            lds[lc].Mu[v][lt] = mu[v];
+            lds[lc].LR[v][lt] = 0.0;
         }
     }
-    wave_lds_sync();
+    sync();
+
+    // ---- the line of this wavefront ----------------------------------------
+    const int t = (int)threadIdx.x % kWave;
+    Lds& s = lds[threadIdx.x / kWave];
+    const int p = position(t);
+    const int li = line_index(min(line0 + (int)threadIdx.x / kWave, a.nlines - 1));
+    const bool line_in = Axis == 0 ? true : (li >= g.ng && li < g.ng + g.nx);
 
     // reconstruction of the cell at p (cells ng-1 .. ng+n along the axis)
     const bool rec_ok = line_in && t >= ORD && t <= kWave - 1 - ORD && (circ || (p >= g.ng - 1 && p <= g.ng + nax));
@@ -127,12 +155,12 @@ __global__ __launch_bounds__(64) void adj_line_kernel(LineArgs a) {
     if (rec_ok) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            auto s = [&](int o) -> double { return sW[v][t + o]; };
-            reconstruct_stencil<R, SL, double>(s, wl[v], wr[v]);
+            auto st = [&](int o) -> double { return s.W[v][t + o]; };
+            reconstruct_stencil<R, SL, double>(st, wl[v], wr[v]);
         }
     }
 #pragma unroll
-    for (int v = 0; v < 4; ++v) sWR[v][t] = wr[v];
+    for (int v = 0; v < 4; ++v) s.WR[v][t] = wr[v];
     wave_lds_sync();
 
     // face at the left edge of p (faces ng .. ng+n): RR of p-1 against RL of p
@@ -141,12 +169,12 @@ __global__ __launch_bounds__(64) void adj_line_kernel(LineArgs a) {
         double wrl[4], lf[4], lrl[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            wrl[v] = sWR[v][t - 1];
-            lf[v] = g.dtdx * (sMu[v][t] - sMu[v][t - 1]);
+            wrl[v] = s.WR[v][t - 1];
+            lf[v] = g.dtdx * (s.Mu[v][t] - s.Mu[v][t - 1]);
         }
         face_vjp<RS, Axis>(g.gamma, wrl, wl, lf, lrl, lL);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) sLR[v][t - 1] = lrl[v];
+        for (int v = 0; v < 4; ++v) s.LR[v][t - 1] = lrl[v];
     }
     wave_lds_sync();
 
@@ -154,28 +182,32 @@ __global__ __launch_bounds__(64) void adj_line_kernel(LineArgs a) {
     // sum of the contributions aimed at it: stencil entry o of the cell in
     // lane t - (o - ORD), read across lanes, summed in order of o
     const bool vjp_ok = rec_ok && t >= ORD + 1 && t <= kWave - 2 - ORD;
-    double lw[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
         double ls[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
         if (vjp_ok) {
             double st[5];
 #pragma unroll
-            for (int o = 0; o < 5; ++o) st[o] = (o >= 2 - ORD && o <= 2 + ORD) ? sW[v][t + o - 2] : 0.0;
+            for (int o = 0; o < 5; ++o) st[o] = (o >= 2 - ORD && o <= 2 + ORD) ? s.W[v][t + o - 2] : 0.0;
             if constexpr (R == Reconstruction::Weno5Z) {
-                weno5z_vjp(st, lL[v], sLR[v][t], ls);
+                weno5z_vjp(st, lL[v], s.LR[v][t], ls);
             } else {
-                reconstruct_vjp_dual<R, SL>(st, lL[v], sLR[v][t], ls);
+                reconstruct_vjp_dual<R, SL>(st, lL[v], s.LR[v][t], ls);
             }
         }
         double sum = 0.0;
 #pragma unroll
         for (int o = 0; o < 2 * ORD + 1; ++o)
             sum += o == ORD ? ls[2] : lane_value(ls[2 - ORD + o], t - (o - ORD));
-        lw[v] = sum;
+        s.WR[v][t] = sum;  // (its face states were read above)
     }
+    sync();
 
-    if (t < HALO || t >= HALO + OUT || p >= (circ ? g.ng + nax : len)) return;
+    // ---- results, by the thread that loaded the cell ------------------------
+    if (lt < HALO || lt >= HALO + OUT || lp >= (circ ? g.ng + nax : len) || line0 + lc >= a.nlines) return;
+    double lw[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) lw[v] = lds[lc].WR[v][lt];
     if constexpr (Axis == 0) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) a.lamx[v * nc + cell] = lw[v];
@@ -284,15 +316,18 @@ __global__ void adj_axpby_kernel(AdjGrid g, double a, const double* __restrict__
 template <RiemannSolver RS, Reconstruction R, SlopeLimiter SL>
 hipError_t stage_impl(const AdjGrid& g, const AdjStage& st, hipStream_t stream) {
     constexpr int OUT = kWave - 2 * (2 * stencil_order(R) + 1);
-    LineArgs a{g, st.q, st.mu, st.lamx, st.nxt, st.acc, st.a_qn, st.a_qs, st.a_l, st.acc_mode, 0, 0, 0};
+    LineArgs a{g, st.q, st.mu, st.lamx, st.nxt, st.acc, st.a_qn, st.a_qs, st.a_l, st.acc_mode, 0, 0, 0, 0};
     const auto per = (int32_t)BoundaryType::Periodic;
     a.circ_x = g.bc[0] == per && g.bc[1] == per;
     a.circ_y = g.bc[2] == per && g.bc[3] == per;
     a.nseg = ((a.circ_x ? g.nx : g.xc) + OUT - 1) / OUT;
-    hipLaunchKernelGGL((adj_line_kernel<R, SL, RS, 0>), dim3(a.nseg * g.ny), dim3(kWave), 0, stream, a);
+    a.nlines = g.ny;
+    hipLaunchKernelGGL((adj_line_kernel<R, SL, RS, 0>), dim3(a.nseg * a.nlines), dim3(kWave), 0, stream, a);
     a.nseg = ((a.circ_y ? g.ny : g.yc) + OUT - 1) / OUT;
-    hipLaunchKernelGGL((adj_line_kernel<R, SL, RS, 1>), dim3(a.nseg * (a.circ_x ? g.nx : g.xc)), dim3(kWave), 0, stream,
-                       a);
+    a.nlines = a.circ_x ? g.nx : g.xc;
+    constexpr int L = kLines<1>;
+    hipLaunchKernelGGL((adj_line_kernel<R, SL, RS, 1>), dim3(a.nseg * ((a.nlines + L - 1) / L)), dim3(kWave * L), 0,
+                       stream, a);
     // ghost cotangents of the non-circular axes into their sources (the
     // ghost entries of a circular axis are never written and stay zero)
     if (!a.circ_y)
