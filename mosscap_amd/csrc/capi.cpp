@@ -193,9 +193,13 @@ void* mh_stream(mh_ctx* ctx) { return ctx ? (void*)ctx->stream : nullptr; }
 int mh_set_user_bc(mh_ctx* ctx, mh_user_bc_fn fn, void* user) {
     if (!ctx) return MH_ERR_INVALID;
     if (ctx->next_stage != 0) return ctx->fail(MH_ERR_INVALID, "a step is in progress (mh_stage)");
+    hipError_t e = hipSetDevice(ctx->device);
+    if (e == hipSuccess) e = ctx->fill_last_input();  // as the stages read them, before the hook
+    if (e != hipSuccess) return ctx->hip_fail(e, "mh_set_user_bc");
     ctx->user_fn = fn;
     ctx->user_data = fn ? user : nullptr;
     ctx->forget_speed();
+    ctx->caller_ghosts = true;
     return MH_OK;
 }
 
@@ -225,9 +229,8 @@ int mh_eos_fields(mh_ctx* ctx, int32_t which, double avg_mass, int32_t ionisatio
     int flag = 0;
     // Steps with ghosts read from their sources leave the ghosts of the
     // intermediate stage inputs unfilled; the fields cover every cell, so
-    // fill them here (plain copies of interior cells, the values those
-    // stages read).
-    e = (k != ctx->cur && ctx->virtual_ghosts()) ? ctx->ghost(k, k, 0) : hipSuccess;
+    // fill them here (the values those stages read).
+    e = k != ctx->cur ? ctx->fill_last_input() : hipSuccess;
     if (e == hipSuccess) e = hipMemsetAsync(ctx->eos_flag, 0, sizeof(int), ctx->stream);
     if (e == hipSuccess) {
         e = ctx->fp32c() ? launch_lte_eos_f32c(ctx->nd, ctx->p32(k), (int)ctx->ncells, prm, ctx->eos_y, ctx->eos_T,
@@ -300,6 +303,7 @@ static int upload_impl(mh_ctx* c, const double* q, hipMemcpyKind kind) {
         if (e == hipSuccess) e = hipMemcpyAsync(c->q64[c->cur], q, bytes, kind, c->stream);
     }
     c->forget_speed();
+    c->caller_ghosts = true;
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return c->hip_fail(e, "mh_upload");
     c->next_stage = 0;
@@ -334,6 +338,7 @@ int mh_fill_bcs(mh_ctx* ctx) {
     ctx->forget_speed();  // a hook may change ghost values; state written through mh_device_state
     if (e == hipSuccess) e = ctx->ghost(ctx->cur, ctx->cur, 0);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) ctx->caller_ghosts = ctx->user_fn != nullptr;
     return e == hipSuccess ? MH_OK : ctx->hip_fail(e, "mh_fill_bcs");
 }
 
@@ -365,6 +370,8 @@ int mh_set_tabulated_eos(mh_ctx* ctx, const mh_lte_table* t) {
     if (!ctx) return MH_ERR_INVALID;
     if (ctx->next_stage != 0) return ctx->fail(MH_ERR_INVALID, "a step is in progress (mh_stage)");
     hipError_t e = hipSetDevice(ctx->device);
+    if (e == hipSuccess) e = ctx->fill_last_input();  // as the stages read them, before the table
+    ctx->caller_ghosts = true;
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     for (double** p : {&ctx->tab_y, &ctx->tab_lT, &ctx->tab_yspace, &ctx->tab_Tspace}) {
         if (*p) hipFree(*p);
@@ -457,6 +464,7 @@ int mh_stage(mh_ctx* ctx, int32_t stage, double dt) {
     hipError_t e = hipSetDevice(ctx->device);
     ctx->forget_speed();
     if (stage == 0) ctx->qn = ctx->cur;
+    ctx->begin_step();
     const int in = ctx->cur;
     const int out = (in == ctx->qn) ? (ctx->qn + 1) % 3 : 3 - in - ctx->qn;
     if (e == hipSuccess) e = ctx->set_dt(dt);
@@ -464,6 +472,7 @@ int mh_stage(mh_ctx* ctx, int32_t stage, double dt) {
     ctx->last_in = in;
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) return ctx->hip_fail(e, "mh_stage");
+    ctx->caller_ghosts = ctx->user_fn != nullptr;
     if (const int rc = tab_check(ctx); rc != MH_OK) return rc;
     ctx->cur = out;
     ctx->next_stage = (stage + 1) % ns;
@@ -482,10 +491,12 @@ int mh_time_step(mh_ctx* ctx, double dt) {
     ctx->forget_speed();
     if (e == hipSuccess) e = ctx->set_dt(dt);
     int nc = ctx->cur;
+    ctx->begin_step();
     if (e == hipSuccess) nc = ctx->enqueue_step(ctx->cur, fold, e);
     if (e == hipSuccess) e = ctx->fill_final(nc);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) return ctx->hip_fail(e, "mh_time_step");
+    ctx->caller_ghosts = ctx->user_fn != nullptr;
     ctx->cur = nc;
     if (const int rc = tab_check(ctx); rc != MH_OK) return rc;
     ctx->amax_valid = fold && !ctx->exposed;
@@ -509,9 +520,11 @@ int mh_run(mh_ctx* ctx, int64_t nsteps, double max_cfl, double* time, double max
         e = launch_clock_start(ctx->clock, clock_fields(ctx, max_cfl, *time, max_time, *prev_output_time, delta),
                                keep_max ? 0 : 1, ctx->stream);
     if (e == hipSuccess && !keep_max) e = ctx->cfl_all(ctx->cur);
+    ctx->begin_step();
     for (int64_t s = 0; s < nsteps && e == hipSuccess; ++s) {
         const int k = ctx->cur;
-        if (use_graph && !ctx->user_fn) {
+        if (use_graph && !ctx->user_fn && !ctx->reads_caller_ghosts()) {
+            ctx->unfilled = ctx->virtual_ghosts();
             if (!ctx->graph[k]) {
                 hipGraph_t g = nullptr;
                 e = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);
@@ -542,6 +555,7 @@ int mh_run(mh_ctx* ctx, int64_t nsteps, double max_cfl, double* time, double max
             e = ctx->finalize(1);
             if (e == hipSuccess) ctx->cur = ctx->enqueue_step(k, true, e);
         }
+        ctx->caller_ghosts = ctx->user_fn != nullptr;
         ctx->steps += 1;
     }
     if (e == hipSuccess && nsteps > 0) e = ctx->fill_final(ctx->cur);
@@ -599,6 +613,7 @@ int mh_autotune(mh_ctx* ctx, int32_t steps, const int32_t* candidates, int32_t* 
     if (ctx->next_stage != 0) return ctx->fail(MH_ERR_INVALID, "a step is in progress (mh_stage)");
     // rows per span; -1: the default layout (march_spans with rows <= 0)
     static const int32_t kDefault[] = {4, 8, 12, 16, 18, 20, 24, 28, 32, 48, 64, -1, 0};
+    const bool own_ghosts = ctx->caller_ghosts;
     const int32_t* cand = candidates ? candidates : kDefault;
     hipError_t e = hipSetDevice(ctx->device);
     // keep the state in a scratch copy and restore it after each trial
@@ -699,6 +714,7 @@ int mh_autotune(mh_ctx* ctx, int32_t steps, const int32_t* candidates, int32_t* 
     }
     ctx->steps = old_steps;
     ctx->cur = start;
+    ctx->caller_ghosts = own_ghosts;
     ctx->forget_speed();  // the slots hold a trial state's maximum
     if (e != hipSuccess) {
         ctx->nspans = old_spans;

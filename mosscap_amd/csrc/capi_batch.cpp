@@ -106,7 +106,7 @@ struct mh_batch {
             g.max_cfl = fin_cfl;
             g.max_time = fin_max_time;
             g.virt = virtual_ghosts() ? 1 : 0;
-            g.per = bdry.xs == (int32_t)BoundaryType::Periodic;
+            g.faces = g.virt ? ghost_faces(bdry.xs, bdry.xe) : 0;
             // Default grid: a wavefront per item, without the grid-stride
             // loop and its prefetch. It takes 42 VGPRs (64 in FP64) instead of
             // 95 (106), so 8 wavefronts reside on a SIMD and hide the loads,

@@ -266,98 +266,125 @@ struct mh_ctx {
             if (r == hipSuccess) r = stage_kernel(src, qn_k, out, kind, reduce, fin);
             return r;
         });
-        if (e != hipSuccess || (!fill && virtual_ghosts())) return e;
+        unfilled = !fill && virtual_ghosts();
+        if (e != hipSuccess || unfilled) return e;
         return ghost(src, out, reduce);
     }
 
-    // Grids whose faces are all periodic or zerograd, with no user_bc hook, no tracer fields and no tabulated EOS (its update runs
-    // over the ghosts of each stage's input): every ghost is a copy of an
-    // interior cell, so the stage kernels read ghost rows, columns and planes
-    // from their sources (StageGrid::virt) and a step needs one ghost fill,
-    // at its end, instead of one per stage (each a graph node and a kernel
-    // boundary). A stage reads the values the reference's fill would have
-    // written (Boundaries.hpp), so the results are the same bits; leaving the
-    // ghosts out of the CFL max changes nothing (they copy interior values).
-    // mh_stage still fills after every stage. The adjoint's recomputation
-    // skips the fills too; its reverse sweep reads ghosts from their sources.
+    // Grids whose faces are all periodic, zerograd, symmetric or wall, with no
+    // user_bc hook and no tabulated EOS (its update runs over the ghosts of
+    // each stage's input): every ghost is a copy of an interior cell, beyond a
+    // wall with the normal velocity negated, so the stage kernels read ghost
+    // rows, columns and planes from their sources (StageGrid::virt) and a step
+    // needs one ghost fill, at its end, instead of one per stage (each a graph
+    // node and a kernel boundary). A stage reads the values the reference's
+    // fill would have written (Boundaries.hpp), so the results are the same
+    // bits; leaving the ghosts out of the CFL max changes nothing (their speed
+    // is their source's). mh_stage still fills after every stage.
     bool virtual_ghosts() const {
+        return !user_fn && !tab_on && ghost_faces(bdry.xs, bdry.xe) >= 0 &&
+               (nd < 2 || ghost_faces(bdry.ys, bdry.ye) >= 0) && (nd < 3 || ghost_faces(bdry.zs, bdry.ze) >= 0);
+    }
+    // 2-D and 3-D grids without tracers, faces periodic or zerograd: their
+    // stages always read ghosts from the sources, and the adjoint's
+    // recomputation (which fills no ghosts then) and reverse sweep do too.
+    bool copy_ghosts() const {
         const auto copy_bc = [](int32_t b) {
             return b == (int32_t)BoundaryType::Periodic || b == (int32_t)BoundaryType::ZeroGrad;
         };
-        return !user_fn && ntr == 0 && !tab_on && copy_bc(bdry.xs) && copy_bc(bdry.xe) &&
-               (nd < 2 || (copy_bc(bdry.ys) && copy_bc(bdry.ye))) &&
-               (nd < 3 || (copy_bc(bdry.zs) && copy_bc(bdry.ze)));
+        return nd > 1 && virtual_ghosts() && ntr == 0 && copy_bc(bdry.xs) && copy_bc(bdry.xe) && copy_bc(bdry.ys) &&
+               copy_bc(bdry.ye) && (nd < 3 || (copy_bc(bdry.zs) && copy_bc(bdry.ze)));
     }
-    void set_virt(StageGrid& g) const {
-        g.virt = virtual_ghosts() ? 1 : 0;
-        g.xper = bdry.xs == (int32_t)BoundaryType::Periodic;
-        g.yper = bdry.ys == (int32_t)BoundaryType::Periodic;
-        g.zper = bdry.zs == (int32_t)BoundaryType::Periodic;
+    // The others do once the library has filled the state's ghosts itself. A
+    // state as the caller left it (an upload, a hook or a write through
+    // mh_device_state, with no mh_fill_bcs after it) keeps the ghosts it came
+    // with for the first stage that reads it.
+    bool caller_ghosts = true;
+    bool reads_caller_ghosts() const { return caller_ghosts && virtual_ghosts() && !copy_ghosts(); }
+    void begin_step() { caller_ghosts = caller_ghosts || exposed; }  // (before each call's first stage)
+    bool virtual_input(int in) const { return virtual_ghosts() && !(in == cur && reads_caller_ghosts()); }
+    // the last step's stage inputs have no ghosts of their own
+    bool unfilled = false;
+    // ... given to those that mh_eos_fields may read of the last stage's input
+    hipError_t fill_last_input() {
+        if (last_in < 0 || last_in == cur || !(unfilled || copy_ghosts())) return hipSuccess;
+        unfilled = false;
+        return ghost(last_in, last_in, 0);
+    }
+    int32_t faces(int axis) const {
+        const int32_t b[6] = {bdry.xs, bdry.xe, bdry.ys, bdry.ye, bdry.zs, bdry.ze};
+        return ghost_faces(b[2 * axis], b[2 * axis + 1]);
+    }
+    void set_virt(StageGrid& g, bool virt) const {
+        g.virt = virt ? 1 : 0;
+        g.xf = faces(0);
+        g.yf = faces(1);
+        g.zf = faces(2);
     }
 
     // 3-D march grid (the interior fold of the CFL max with `reduce`)
-    StageGrid grid3(int kind, int reduce) const {
+    StageGrid grid3(int kind, int reduce, bool virt) const {
         StageGrid g{sz.xc, sz.yc, sz.ng, sz.xc - 2 * sz.ng, sz.yc - 2 * sz.ng, strips, nspans, kind, reduce};
         g.zc = sz.zc;
         g.nz = sz.zc - 2 * sz.ng;
         g.flat = flat;
-        set_virt(g);
+        set_virt(g, virt);
         return g;
     }
 
     hipError_t stage_kernel(int in, int qn_k, int out, int kind, int reduce, int fin = 0) {
         hipError_t e;
-        const TracerGrid tg{sz.xc, sz.yc, sz.ng, sz.xc - 2 * sz.ng, sz.yc - 2 * sz.ng, ntr, kind};
+        const bool virt = virtual_input(in);
+        const TracerGrid tg{sz.xc, sz.yc, sz.ng, sz.xc - 2 * sz.ng, sz.yc - 2 * sz.ng, ntr, kind,
+                            virt ? 1 : 0, faces(0), faces(1)};
         if (fp32c()) {
             FormF32c::Ptrs p{p32(in), p32(qn_k), p32(out), &clock->dt, dx, gamma, gamma - 1.0,
                              amax_slots(clock), floor_hits, opt.rho_floor, opt.p_floor, frx32, fry32,
                              gravity, grav[0], grav[1]};
             if (nd == 2) {
                 StageGrid g{sz.xc, sz.yc, sz.ng, sz.xc - 2 * sz.ng, sz.yc - 2 * sz.ng, strips, nspans, kind, reduce};
-                set_virt(g);
+                set_virt(g, virt);
                 g.fin = fin;
                 g.clock = clock;
                 e = launch_stage2d_f32c(sch, g, p, stream);
                 if (e == hipSuccess && ntr > 0) e = launch_tracer_f32c(sch, tg, p, wtr32, stream);
             } else if (nd == 3) {
                 p.gz = grav[2];
-                e = launch_stage3d_f32c(sch, grid3(kind, reduce), p, dz32, stream);
+                e = launch_stage3d_f32c(sch, grid3(kind, reduce, virt), p, dz32, stream);
             } else {
-                e = launch_stage1d_f32c(sch, kind, reduce, sz.xc, sz.ng, p, stream, virtual_ghosts() ? 1 : 0,
-                                        bdry.xs == (int32_t)BoundaryType::Periodic);
+                e = launch_stage1d_f32c(sch, kind, reduce, sz.xc, sz.ng, p, stream, virt ? 1 : 0, faces(0));
             }
         } else {
             FormF64::Ptrs p{p64(in), p64(qn_k), p64(out), &clock->dt, dx, gamma, amax_slots(clock), nullptr,
                             frx64, fry64, gravity, grav[0], grav[1]};
             if (nd == 2) {
                 StageGrid g{sz.xc, sz.yc, sz.ng, sz.xc - 2 * sz.ng, sz.yc - 2 * sz.ng, strips, nspans, kind, reduce};
-                set_virt(g);
+                set_virt(g, virt);
                 g.fin = fin;
                 g.clock = clock;
                 e = launch_stage2d_f64(sch, g, p, stream);
                 if (e == hipSuccess && ntr > 0) e = launch_tracer_f64(sch, tg, p, wtr64, stream);
             } else if (nd == 3) {
                 p.gz = grav[2];
-                e = launch_stage3d_f64(sch, grid3(kind, reduce), p, dz64, stream);
+                e = launch_stage3d_f64(sch, grid3(kind, reduce, virt), p, dz64, stream);
             } else {
-                e = launch_stage1d_f64(sch, kind, reduce, sz.xc, sz.ng, p, stream, virtual_ghosts() ? 1 : 0,
-                                       bdry.xs == (int32_t)BoundaryType::Periodic);
+                e = launch_stage1d_f64(sch, kind, reduce, sz.xc, sz.ng, p, stream, virt ? 1 : 0, faces(0));
             }
         }
         return e;
     }
 
     // FP64 stage between arbitrary device buffers (adjoint recomputation).
-    // dt_dev: the step's dt in device memory. With virtual_ghosts() the
+    // dt_dev: the step's dt in device memory. With copy_ghosts() the
     // input's ghosts are read from their sources and the output's are left
     // unfilled (the reverse sweep reads them the same way).
     hipError_t stage_ptr(const double* in, const double* qn_p, double* out, int kind, const double* dt_dev) {
         FormF64::Ptrs p{FormF64::Planes{(double*)in}, FormF64::Planes{(double*)qn_p}, FormF64::Planes{out}, dt_dev,
                         dx, gamma, amax_slots(clock), nullptr, nullptr, nullptr, gravity, grav[0], grav[1]};
         StageGrid g{sz.xc, sz.yc, sz.ng, sz.xc - 2 * sz.ng, sz.yc - 2 * sz.ng, strips, nspans, kind, 0};
-        set_virt(g);
+        set_virt(g, copy_ghosts());
         hipError_t e = launch_stage2d_f64(sch, g, p, stream);  // the adjoint is 2-D
-        if (e != hipSuccess || virtual_ghosts()) return e;
+        if (e != hipSuccess || copy_ghosts()) return e;
         return launch_ghost_f64(nd, ghost_grid(0), FormF64::Planes{(double*)in}, FormF64::Planes{out}, nullptr, stream);
     }
 

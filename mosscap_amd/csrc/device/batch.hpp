@@ -25,7 +25,7 @@ struct BatchArrays {
 
 struct BatchGrid {
     int32_t ng, nitems, nprob, kind, reduce_dt;
-    int32_t virt, per;  // ghosts read from their sources (periodic `per`, else zerograd); no fill per stage
+    int32_t virt, faces;  // ghosts read from their sources (ghost_faces of the ends); no fill per stage
     // The step's per-problem clock work folded into its stages (graph-replayed
     // persistent steps of three or more stages): 1 = this first stage takes
     // each problem's dt from its CFL max and clock itself and the wave with
@@ -67,7 +67,6 @@ __device__ inline void batch_stage(const BatchGrid& g, const typename Form::Ptrs
     __shared__ T lds[3 * (kWave + 2 * ORD)];
     const int lane = threadIdx.x & 63;
     const int virt = Form::kVirtualGhosts ? g.virt : 0;
-    const bool per = g.per != 0;
     unsigned int hits = 0;
     // Consecutive items go to one XCD: a segment's 62 cells are not a whole
     // number of cache lines, so its neighbours read and write the lines at its
@@ -77,7 +76,7 @@ __device__ inline void batch_stage(const BatchGrid& g, const typename Form::Ptrs
     const Item* items = reinterpret_cast<const Item*>(b.items);
     Item w = uniform_load(items, it < g.nitems ? it : 0);
     SegRaw<Form> cur;
-    if (it < g.nitems) seg_load<Form, R>(p, g.kind, w.z, w.w, g.ng, w.w - 2 * g.ng, w.y, virt, per, cur);
+    if (it < g.nitems) seg_load<Form, R>(p, g.kind, w.z, w.w, g.ng, w.w - 2 * g.ng, w.y, virt, g.faces, cur);
     for (; it < g.nitems; it += gridDim.x) {
         const int pr = w.x, i0 = w.y, base = w.z, xc = w.w;
         double dt_step;
@@ -93,7 +92,7 @@ __device__ inline void batch_stage(const BatchGrid& g, const typename Form::Ptrs
         SegRaw<Form> nxt = cur;
         if (Loop && nit < g.nitems) {
             w = uniform_load(items, nit);
-            seg_load<Form, R>(p, g.kind, w.z, w.w, g.ng, w.w - 2 * g.ng, w.y, virt, per, nxt);
+            seg_load<Form, R>(p, g.kind, w.z, w.w, g.ng, w.w - 2 * g.ng, w.y, virt, g.faces, nxt);
         }
         if (i0 == g.ng && lane == 0) {  // the wave with the problem's first segment
             if (g.fin == 1) b.dt[pr] = dt_step;
@@ -106,7 +105,7 @@ __device__ inline void batch_stage(const BatchGrid& g, const typename Form::Ptrs
         const T dtdx = dt / (T)dx;
         double amax = 0.0;
         seg_compute<Form, R, SL, RS>(p, g.kind, g.reduce_dt, base, xc, g.ng, xc - 2 * g.ng, i0, dtdx, dt, lds, amax,
-                                     hits, cur);
+                                     hits, cur, virt, g.faces);
         if (g.reduce_dt) {
             const uint64_t m = wave_max_u64(__builtin_bit_cast(uint64_t, amax));
             if (lane == 0) atomicMax(&b.amax[pr], (unsigned long long)m);

@@ -107,10 +107,55 @@ __host__ __device__ inline int ghost_source(int g, int dims, int ng, BoundaryTyp
     }
 }
 
-// Source index of index i of an axis with n interior cells and ng ghosts on
-// each side when its ghosts are copies: ghost_source() for Periodic and
-// ZeroGrad; interior indices map to themselves. Readers of a state whose
-// ghosts were not filled use it in place of the fill.
+// The two faces of an axis whose ghosts stage kernels read from their sources:
+// low face + 4 * high face, each one of these. (A diode face changes the
+// energy too, a constant one has no source and a user_fn one is the caller's.)
+enum GhostFace : int32_t { kFaceZeroGrad = 0, kFacePeriodic = 1, kFaceSymmetric = 2, kFaceWall = 3 };
+__host__ inline int32_t ghost_faces(int32_t lo, int32_t hi) {  // BoundaryType of the faces; -1: not such faces
+    const auto face = [](int32_t b) -> int32_t {
+        switch ((BoundaryType)b) {
+            case BoundaryType::ZeroGrad: return kFaceZeroGrad;
+            case BoundaryType::Periodic: return kFacePeriodic;
+            case BoundaryType::Symmetric: return kFaceSymmetric;
+            case BoundaryType::Wall: return kFaceWall;
+            default: return -1;
+        }
+    };
+    return face(lo) < 0 || face(hi) < 0 ? -1 : face(lo) + 4 * face(hi);
+}
+// ghost_source() of index i of an axis with n interior cells, ng ghosts on
+// each side and these faces; interior indices map to themselves.
+__host__ __device__ inline int face_source(int i, int n, int ng, int32_t faces) {
+    if (i < ng) {
+        const int f = faces & 3;
+        return f == kFacePeriodic ? i + n : f == kFaceZeroGrad ? ng : 2 * ng - 1 - i;
+    }
+    if (i >= ng + n) {
+        const int f = faces >> 2;
+        return f == kFacePeriodic ? i - n : f == kFaceZeroGrad ? ng + n - 1 : 2 * (ng + n) - 1 - i;
+    }
+    return i;
+}
+// ... and whether the ghost's velocity along the axis is its source's negated
+// (Boundaries.hpp:83-88). Negating a velocity after cons->prim gives the bits
+// of cons->prim of the negated momentum.
+__host__ __device__ inline bool face_flips(int i, int n, int ng, int32_t faces) {
+    return (i < ng && (faces & 3) == kFaceWall) || (i >= ng + n && (faces >> 2) == kFaceWall);
+}
+
+// All axes' faces are copies, the two of an axis alike: copy_ghost_source()
+// with `periodic` = the axis' faces are kAxisPeriodic.
+constexpr int32_t kAxisPeriodic = 5 * kFacePeriodic;
+__host__ __device__ inline bool axis_copies(int32_t faces) { return faces == 0 || faces == kAxisPeriodic; }
+// A velocity as read through face_source(): flip = face_flips().
+__host__ __device__ inline float flip_sign(float x, bool flip) {
+    return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) ^ (flip ? 0x80000000u : 0u));
+}
+__host__ __device__ inline double flip_sign(double x, bool flip) {
+    return __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, x) ^ ((uint64_t)(flip ? 0x80000000u : 0u) << 32));
+}
+
+// face_source() of an axis whose faces are both periodic or both zero-gradient.
 __host__ __device__ inline int copy_ghost_source(int i, int n, int ng, bool periodic) {
     if (i < ng) return periodic ? i + n : ng;
     if (i >= ng + n) return periodic ? i - n : ng + n - 1;

@@ -26,10 +26,10 @@ struct ZSweepGrid {
     int32_t xc, yc, zc, ng;
     int32_t nx, ny, nz;
     int32_t kchunk;  // interior planes per thread (blockIdx.y selects the chunk)
-    int32_t virt = 0, zper = 0;  // ghost planes read from their sources (StageGrid::virt)
+    int32_t virt = 0, zf = 0;  // ghost planes read from their sources (StageGrid::virt)
 };
 
-template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS>
+template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS, bool Copies>
 __device__ inline void zsweep_column(const ZSweepGrid& g, const typename Form::Ptrs& p, typename Form::real* dz) {
     using T = typename Form::real;
     using Raw = typename Form::raw;
@@ -52,11 +52,14 @@ __device__ inline void zsweep_column(const ZSweepGrid& g, const typename Form::P
 
     T win[WIN][NV];
     auto load = [&](int k, T (&w)[NV]) {
-        const int ks = (Form::kVirtualGhosts && g.virt) ? copy_ghost_source(k, g.nz, g.ng, g.zper) : k;
+        int ks = k;
+        if (Form::kVirtualGhosts && g.virt)
+            ks = Copies ? copy_ghost_source(k, g.nz, g.ng, g.zf == kAxisPeriodic) : face_source(k, g.nz, g.ng, g.zf);
         Raw q[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) q[v] = Form::get(p.qs, v * vs + ks * pl + base);
         Form::template to_prim_nd<ND>(p, q, w);
+        if constexpr (!Copies) w[3] = flip_sign(w[3], Form::kVirtualGhosts && g.virt && face_flips(k, g.nz, g.ng, g.zf));
     };
     auto recon = [&](T (&wl)[NV], T (&wr)[NV]) {
 #pragma unroll

@@ -23,6 +23,7 @@ struct TracerGrid {
     int32_t xc, yc, ng, nx, ny;
     int32_t ntr;   // tracer count; planes 4 .. 3+ntr of the state
     int32_t kind;  // StageKind
+    int32_t virt, xf, yf;  // ghosts read from their sources (StageGrid::virt), where they are not filled
 };
 
 // W_t = Q_t * (1/rho) on every cell (ghosts included), FP64 reciprocal as in
@@ -34,9 +35,12 @@ __global__ __launch_bounds__(256) void tracer_prim_kernel(TracerGrid g, typename
     const int plane = g.xc * g.yc;
     const int cell = blockIdx.x * blockDim.x + threadIdx.x;
     if (cell >= plane) return;
-    const double inv_rho = 1.0 / Form::value(Form::get(qs, cell));
+    // (neither a density nor a tracer changes its sign beyond a wall)
+    const int from = g.virt ? face_source(cell / g.xc, g.ny, g.ng, g.yf) * g.xc + face_source(cell % g.xc, g.nx, g.ng, g.xf)
+                            : cell;
+    const double inv_rho = 1.0 / Form::value(Form::get(qs, from));
     for (int k = 0; k < g.ntr; ++k) {
-        const double q = Form::value(Form::get(qs, (4 + k) * plane + cell));
+        const double q = Form::value(Form::get(qs, (4 + k) * plane + from));
         wtr[k * plane + cell] = (T)(q * inv_rho);
     }
 }

@@ -30,8 +30,8 @@ hipError_t launch_stage2d_f32c(const Schemes& s, const StageGrid& g, const FormF
 }
 
 hipError_t launch_stage1d_f32c(const Schemes& s, int kind, int reduce_dt, int xc, int ng, const FormF32c::Ptrs& p,
-                               hipStream_t st, int virt, int per) {
-    return launch_stage1d_impl<FormF32c>(s, kind, reduce_dt, xc, ng, p, st, virt, per);
+                               hipStream_t st, int virt, int32_t faces) {
+    return launch_stage1d_impl<FormF32c>(s, kind, reduce_dt, xc, ng, p, st, virt, faces);
 }
 
 hipError_t launch_tracer_f32c(const Schemes& s, const TracerGrid& g, const FormF32c::Ptrs& p,

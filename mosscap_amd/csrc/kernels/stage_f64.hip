@@ -20,8 +20,8 @@ hipError_t launch_stage2d_f64(const Schemes& s, const StageGrid& g, const FormF6
 }
 
 hipError_t launch_stage1d_f64(const Schemes& s, int kind, int reduce_dt, int xc, int ng, const FormF64::Ptrs& p,
-                              hipStream_t st, int virt, int per) {
-    return launch_stage1d_impl<FormF64>(s, kind, reduce_dt, xc, ng, p, st, virt, per);
+                              hipStream_t st, int virt, int32_t faces) {
+    return launch_stage1d_impl<FormF64>(s, kind, reduce_dt, xc, ng, p, st, virt, faces);
 }
 
 hipError_t launch_tracer_f64(const Schemes& s, const TracerGrid& g, const FormF64::Ptrs& p,

@@ -21,18 +21,18 @@
 
 namespace mh {
 
-template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS, int Inst>
+template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS, int Inst, bool Copies>
 __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(Inst == kStageExtras   ? MH_STAGE_WAVES_EXTRAS
                                    : Inst == kStageFloors ? MH_STAGE_WAVES_FLOORS
                                                           : MH_STAGE_WAVES_PER_EU)))
 void stage2d_kernel(StageGrid g, typename Form::Ptrs p) {
-    stage2d_march<Form, R, SL, RS, 2, Inst>(g, p);
+    stage2d_march<Form, R, SL, RS, 2, Inst, Copies>(g, p);
 }
 
 struct Stage1dGrid {
     int32_t xc, ng, nx, kind, reduce_dt;
-    int32_t virt, per;  // ghosts read from their sources (StageGrid::virt; periodic `per`, else zerograd)
+    int32_t virt, faces;  // ghosts read from their sources (StageGrid::virt, ghost_faces of the ends)
 };
 
 template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS>
@@ -46,7 +46,7 @@ __global__ __launch_bounds__(64) void stage1d_kernel(Stage1dGrid g, typename For
     double amax = 0.0;
     unsigned int hits = 0;
     stage1d_segment<Form, R, SL, RS>(p, g.kind, g.reduce_dt, 0, g.xc, g.ng, g.nx, i0, dtdx, dt, lds, amax, hits,
-                                     Form::kVirtualGhosts ? g.virt : 0, g.per != 0);
+                                     Form::kVirtualGhosts ? g.virt : 0, g.faces);
     if (g.reduce_dt) {
         const uint64_t m = wave_max_u64(__builtin_bit_cast(uint64_t, amax));
         if (threadIdx.x == 0) atomicMax(p.amax_bits, (unsigned long long)m);
@@ -64,12 +64,12 @@ using Stage1dFn = void (*)(Stage1dGrid, typename Form::Ptrs);
 
 template <class Form, Reconstruction R, SlopeLimiter SL>
 struct SolverPick {
-    template <int Inst>
+    template <int Inst, bool Copies>
     static Stage2dFn<Form> two(RiemannSolver rs) {
         switch (rs) {
-            case RiemannSolver::Rusanov: return stage2d_kernel<Form, R, SL, RiemannSolver::Rusanov, Inst>;
-            case RiemannSolver::Hll: return stage2d_kernel<Form, R, SL, RiemannSolver::Hll, Inst>;
-            default: return stage2d_kernel<Form, R, SL, RiemannSolver::Hllc, Inst>;
+            case RiemannSolver::Rusanov: return stage2d_kernel<Form, R, SL, RiemannSolver::Rusanov, Inst, Copies>;
+            case RiemannSolver::Hll: return stage2d_kernel<Form, R, SL, RiemannSolver::Hll, Inst, Copies>;
+            default: return stage2d_kernel<Form, R, SL, RiemannSolver::Hllc, Inst, Copies>;
         }
     }
     static Stage1dFn<Form> one(RiemannSolver rs) {
@@ -115,12 +115,14 @@ hipError_t launch_stage2d_impl(const Schemes& s, const StageGrid& g, const typen
     const bool big = (int64_t)4 * g.xc * g.yc * Form::kElem >= ((int64_t)1 << 31);
     const bool extras = p.gravity != 0 || p.frx != nullptr || p.fry != nullptr || big;
     const bool floors = Form::floors_on(p);
+    const bool copies = copy_stage_ghosts(g);
     auto pick = [&]<Reconstruction R, SlopeLimiter SL>() -> Stage2dFn<Form> {
-        if (extras) return SolverPick<Form, R, SL>::template two<kStageExtras>(s.solver);
+        using P = SolverPick<Form, R, SL>;
+        if (extras) return copies ? P::template two<kStageExtras, true>(s.solver) : P::template two<kStageExtras, false>(s.solver);
         if constexpr (Form::kHasFloors) {
-            if (floors) return SolverPick<Form, R, SL>::template two<kStageFloors>(s.solver);
+            if (floors) return copies ? P::template two<kStageFloors, true>(s.solver) : P::template two<kStageFloors, false>(s.solver);
         }
-        return SolverPick<Form, R, SL>::template two<kStagePlain>(s.solver);
+        return copies ? P::template two<kStagePlain, true>(s.solver) : P::template two<kStagePlain, false>(s.solver);
     };
     Stage2dFn<Form> fn = pick_scheme<Form>(s, pick);
     hipLaunchKernelGGL(fn, dim3((unsigned)(g.strips * g.nspans)), dim3(kWave), 0, st, g, p);
@@ -129,28 +131,28 @@ hipError_t launch_stage2d_impl(const Schemes& s, const StageGrid& g, const typen
 
 template <class Form>
 hipError_t launch_stage1d_impl(const Schemes& s, int kind, int reduce_dt, int xc, int ng,
-                               const typename Form::Ptrs& p, hipStream_t st, int virt, int per) {
+                               const typename Form::Ptrs& p, hipStream_t st, int virt, int32_t faces) {
     const int nx = xc - 2 * ng;
     if (nx < 1 || ng < min_ghost_cells(s.recon)) return hipErrorInvalidValue;
     auto pick = [&]<Reconstruction R, SlopeLimiter SL>() { return SolverPick<Form, R, SL>::one(s.solver); };
     Stage1dFn<Form> fn = pick_scheme<Form>(s, pick);
-    const Stage1dGrid g{xc, ng, nx, kind, reduce_dt, virt, per};
+    const Stage1dGrid g{xc, ng, nx, kind, reduce_dt, virt, faces};
     const int segs = (nx + kStripOut - 1) / kStripOut;
     hipLaunchKernelGGL(fn, dim3((unsigned)segs), dim3(kWave), 0, st, g, p);
     return hipGetLastError();
 }
 
 #ifdef MH_STAGE3D_INSTANCES
-template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS, bool Extras>
+template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS, bool Extras, bool Copies>
 __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(Extras ? MH_STAGE_WAVES_EXTRAS : MH_STAGE_WAVES_PER_EU)))
 void stage3d_kernel(StageGrid g, typename Form::Ptrs p) {
-    stage2d_march<Form, R, SL, RS, 3, Extras ? kStageExtras : kStagePlain>(g, p);
+    stage2d_march<Form, R, SL, RS, 3, Extras ? kStageExtras : kStagePlain, Copies>(g, p);
 }
 
-template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS>
+template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS, bool Copies>
 __global__ __launch_bounds__(128) void zsweep_kernel(ZSweepGrid g, typename Form::Ptrs p, typename Form::real* dz) {
-    zsweep_column<Form, R, SL, RS>(g, p, dz);
+    zsweep_column<Form, R, SL, RS, Copies>(g, p, dz);
 }
 
 template <class Form>
@@ -163,29 +165,36 @@ hipError_t launch_stage3d_impl(const Schemes& s, const StageGrid& g, const typen
     const MarchColumns cols = march_columns(g.nx, g.nz, 3, s.recon, sizeof(typename Form::real) == 8);
     if (g.strips != cols.strips || g.flat != cols.flat) return hipErrorInvalidValue;
     using ZFn = void (*)(ZSweepGrid, typename Form::Ptrs, typename Form::real*);
-    auto zpick = [&]<Reconstruction R, SlopeLimiter SL>() -> ZFn {
+    const bool copies = copy_stage_ghosts(g);
+    auto zsolver = [&]<Reconstruction R, SlopeLimiter SL, bool Copies>() -> ZFn {
         switch (s.solver) {
-            case RiemannSolver::Rusanov: return zsweep_kernel<Form, R, SL, RiemannSolver::Rusanov>;
-            case RiemannSolver::Hll: return zsweep_kernel<Form, R, SL, RiemannSolver::Hll>;
-            default: return zsweep_kernel<Form, R, SL, RiemannSolver::Hllc>;
+            case RiemannSolver::Rusanov: return zsweep_kernel<Form, R, SL, RiemannSolver::Rusanov, Copies>;
+            case RiemannSolver::Hll: return zsweep_kernel<Form, R, SL, RiemannSolver::Hll, Copies>;
+            default: return zsweep_kernel<Form, R, SL, RiemannSolver::Hllc, Copies>;
         }
+    };
+    auto zpick = [&]<Reconstruction R, SlopeLimiter SL>() -> ZFn {
+        return copies ? zsolver.template operator()<R, SL, true>() : zsolver.template operator()<R, SL, false>();
     };
     // plain instance (buffer addressing, no source or floors) unless gravity
     // or the floors are on or a byte offset could pass 2^31
     const bool big = (int64_t)5 * g.xc * g.yc * g.zc * Form::kElem >= ((int64_t)1 << 31);
     const bool extras = p.gravity != 0 || Form::floors_on(p) || big;
-    auto mpick = [&]<Reconstruction R, SlopeLimiter SL>() -> Stage2dFn<Form> {
+    auto msolver = [&]<Reconstruction R, SlopeLimiter SL, bool Copies>() -> Stage2dFn<Form> {
         switch (s.solver) {
             case RiemannSolver::Rusanov:
-                return extras ? stage3d_kernel<Form, R, SL, RiemannSolver::Rusanov, true>
-                              : stage3d_kernel<Form, R, SL, RiemannSolver::Rusanov, false>;
+                return extras ? stage3d_kernel<Form, R, SL, RiemannSolver::Rusanov, true, Copies>
+                              : stage3d_kernel<Form, R, SL, RiemannSolver::Rusanov, false, Copies>;
             case RiemannSolver::Hll:
-                return extras ? stage3d_kernel<Form, R, SL, RiemannSolver::Hll, true>
-                              : stage3d_kernel<Form, R, SL, RiemannSolver::Hll, false>;
+                return extras ? stage3d_kernel<Form, R, SL, RiemannSolver::Hll, true, Copies>
+                              : stage3d_kernel<Form, R, SL, RiemannSolver::Hll, false, Copies>;
             default:
-                return extras ? stage3d_kernel<Form, R, SL, RiemannSolver::Hllc, true>
-                              : stage3d_kernel<Form, R, SL, RiemannSolver::Hllc, false>;
+                return extras ? stage3d_kernel<Form, R, SL, RiemannSolver::Hllc, true, Copies>
+                              : stage3d_kernel<Form, R, SL, RiemannSolver::Hllc, false, Copies>;
         }
+    };
+    auto mpick = [&]<Reconstruction R, SlopeLimiter SL>() -> Stage2dFn<Form> {
+        return copies ? msolver.template operator()<R, SL, true>() : msolver.template operator()<R, SL, false>();
     };
     // z sweep: each thread walks a chunk of the planes, columns of the interior
     // across the grid's x; a chunk's prologue (its window of planes, the first
@@ -195,7 +204,7 @@ hipError_t launch_stage3d_impl(const Schemes& s, const StageGrid& g, const typen
     const int chunks = split_marches(2 * (int64_t)blocks, g.nz, 1.5, sizeof(typename Form::real) == 8);
     ZSweepGrid zg{g.xc, g.yc, g.zc, g.ng, g.nx, g.ny, g.nz, (g.nz + chunks - 1) / chunks};
     zg.virt = g.virt;
-    zg.zper = g.zper;
+    zg.zf = g.zf;
     hipLaunchKernelGGL(pick_scheme<Form>(s, zpick), dim3((unsigned)blocks, (unsigned)chunks), dim3(128), 0, st, zg, p,
                        dz);
     typename Form::Ptrs pm = p;

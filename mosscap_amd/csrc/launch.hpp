@@ -71,11 +71,11 @@ hipError_t launch_stage3d_f64(const Schemes& s, const StageGrid& g, const FormF6
 hipError_t launch_stage3d_f32c(const Schemes& s, const StageGrid& g, const FormF32c::Ptrs& p, float* dz,
                                hipStream_t st);
 // 1-D stage over one row of xc cells (ng ghosts each side); virt: ghosts read
-// from their sources, per: periodic, else zerograd.
+// from their sources, faces: ghost_faces of the ends.
 hipError_t launch_stage1d_f64(const Schemes& s, int kind, int reduce_dt, int xc, int ng, const FormF64::Ptrs& p,
-                              hipStream_t st, int virt = 0, int per = 0);
+                              hipStream_t st, int virt = 0, int32_t faces = 0);
 hipError_t launch_stage1d_f32c(const Schemes& s, int kind, int reduce_dt, int xc, int ng, const FormF32c::Ptrs& p,
-                               hipStream_t st, int virt = 0, int per = 0);
+                               hipStream_t st, int virt = 0, int32_t faces = 0);
 
 // Tracer planes of a 2-D stage (p.frx / p.fry hold the stage's density fluxes).
 hipError_t launch_tracer_f64(const Schemes& s, const TracerGrid& g, const FormF64::Ptrs& p, double* wtr,
