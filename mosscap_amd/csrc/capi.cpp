@@ -144,11 +144,9 @@ int mh_create(const mh_grid_size* sz, double dx, const mh_grid_loc* loc, const m
         if (num_tracers > 0 && c->fp32c()) {
             want(c->frx32, cells * r, false);
             want(c->fry32, cells * r, false);
-            want(c->wtr32, cells * num_tracers * r, false);
         } else if (num_tracers > 0) {
             want(c->frx64, cells * r, false);
             want(c->fry64, cells * r, false);
-            want(c->wtr64, cells * num_tracers * r, false);
         }
         if (num_dim == 3 && c->fp32c()) want(c->dz32, cells * 5 * r, false);
         else if (num_dim == 3) want(c->dz64, cells * 5 * r, false);

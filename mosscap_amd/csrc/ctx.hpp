@@ -56,10 +56,8 @@ struct mh_ctx {
     double grav[3] = {0.0, 0.0, 0.0};
     double* frx64 = nullptr;         // tracers: density fluxes of the stage (FP64 form)
     double* fry64 = nullptr;
-    double* wtr64 = nullptr;         // tracers: mass fractions of the stage input
     float* frx32 = nullptr;          // ... compensated form
     float* fry32 = nullptr;
-    float* wtr32 = nullptr;
     double* dz64 = nullptr;          // 3-D: z flux differences of the stage (FP64 form)
     float* dz32 = nullptr;           // ... compensated form
     mh_grid_size sz{};
@@ -335,7 +333,7 @@ struct mh_ctx {
     hipError_t stage_kernel(int in, int qn_k, int out, int kind, int reduce, int fin = 0) {
         hipError_t e;
         const bool virt = virtual_input(in);
-        const TracerGrid tg{sz.xc, sz.yc, sz.ng, sz.xc - 2 * sz.ng, sz.yc - 2 * sz.ng, ntr, kind,
+        const TracerGrid tg{sz.xc, sz.yc, sz.ng, sz.xc - 2 * sz.ng, sz.yc - 2 * sz.ng, ntr, kind, 0, 0,
                             virt ? 1 : 0, faces(0), faces(1)};
         if (fp32c()) {
             FormF32c::Ptrs p{p32(in), p32(qn_k), p32(out), &clock->dt, dx, gamma, gamma - 1.0,
@@ -347,7 +345,7 @@ struct mh_ctx {
                 g.fin = fin;
                 g.clock = clock;
                 e = launch_stage2d_f32c(sch, g, p, stream);
-                if (e == hipSuccess && ntr > 0) e = launch_tracer_f32c(sch, tg, p, wtr32, stream);
+                if (e == hipSuccess && ntr > 0) e = launch_tracer_f32c(sch, tg, p, stream);
             } else if (nd == 3) {
                 p.gz = grav[2];
                 e = launch_stage3d_f32c(sch, grid3(kind, reduce, virt), p, dz32, stream);
@@ -363,7 +361,7 @@ struct mh_ctx {
                 g.fin = fin;
                 g.clock = clock;
                 e = launch_stage2d_f64(sch, g, p, stream);
-                if (e == hipSuccess && ntr > 0) e = launch_tracer_f64(sch, tg, p, wtr64, stream);
+                if (e == hipSuccess && ntr > 0) e = launch_tracer_f64(sch, tg, p, stream);
             } else if (nd == 3) {
                 p.gz = grav[2];
                 e = launch_stage3d_f64(sch, grid3(kind, reduce, virt), p, dz64, stream);
@@ -483,8 +481,8 @@ struct mh_ctx {
         tab_neg = nullptr;
         dz64 = nullptr;
         dz32 = nullptr;
-        frx64 = fry64 = wtr64 = nullptr;
-        frx32 = fry32 = wtr32 = nullptr;
+        frx64 = fry64 = nullptr;
+        frx32 = fry32 = nullptr;
         eos_y = eos_T = nullptr;
         eos_flag = nullptr;
         if (clock_host) hipHostFree(clock_host);

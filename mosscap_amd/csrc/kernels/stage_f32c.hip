@@ -35,8 +35,8 @@ hipError_t launch_stage1d_f32c(const Schemes& s, int kind, int reduce_dt, int xc
 }
 
 hipError_t launch_tracer_f32c(const Schemes& s, const TracerGrid& g, const FormF32c::Ptrs& p,
-                              FormF32c::real* wtr, hipStream_t st) {
-    return launch_tracer_impl<FormF32c>(s, g, p, wtr, st);
+                              hipStream_t st) {
+    return launch_tracer_impl<FormF32c>(s, g, p, st);
 }
 
 }  // namespace mh

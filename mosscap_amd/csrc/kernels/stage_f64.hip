@@ -25,8 +25,8 @@ hipError_t launch_stage1d_f64(const Schemes& s, int kind, int reduce_dt, int xc,
 }
 
 hipError_t launch_tracer_f64(const Schemes& s, const TracerGrid& g, const FormF64::Ptrs& p,
-                              FormF64::real* wtr, hipStream_t st) {
-    return launch_tracer_impl<FormF64>(s, g, p, wtr, st);
+                              hipStream_t st) {
+    return launch_tracer_impl<FormF64>(s, g, p, st);
 }
 
 }  // namespace mh

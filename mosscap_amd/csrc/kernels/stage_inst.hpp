@@ -215,21 +215,21 @@ hipError_t launch_stage3d_impl(const Schemes& s, const StageGrid& g, const typen
 }
 #endif
 
-// Tracer planes of one 2-D stage (after the hydro stage stored the density
-// fluxes): W_t of the stage input, then the interior update.
+// Tracer planes of one 2-D stage, after the hydro stage stored the density
+// fluxes. A span's prologue (its window of rows, two reconstructions) is worth
+// two rows.
 template <class Form>
-hipError_t launch_tracer_impl(const Schemes& s, const TracerGrid& g, const typename Form::Ptrs& p,
-                              typename Form::real* wtr, hipStream_t st) {
+hipError_t launch_tracer_impl(const Schemes& s, TracerGrid g, const typename Form::Ptrs& p, hipStream_t st) {
     if (g.ntr < 1 || g.nx < 1 || g.ny < 1 || g.ng < min_ghost_cells(s.recon) || g.xc != g.nx + 2 * g.ng ||
-        g.yc != g.ny + 2 * g.ng || !wtr || !p.frx || !p.fry)
+        g.yc != g.ny + 2 * g.ng || !p.frx || !p.fry)
         return hipErrorInvalidValue;
-    const int cells = g.xc * g.yc, inner = g.nx * g.ny;
-    hipLaunchKernelGGL(tracer_prim_kernel<Form>, dim3((cells + 255) / 256), dim3(256), 0, st, g, p.qs, wtr);
-    using Fn = void (*)(TracerGrid, typename Form::Ptrs, const typename Form::real*, const typename Form::real*,
-                        const typename Form::real*);
+    const int outs = kWave - 2 * (stencil_order(s.recon) + 1);
+    g.strips = (g.nx + outs - 1) / outs;
+    g.nspans = split_marches((int64_t)g.strips * g.ntr, g.ny, 2.0, sizeof(typename Form::real) == 8);
+    using Fn = void (*)(TracerGrid, typename Form::Ptrs);
     auto pick = [&]<Reconstruction R, SlopeLimiter SL>() -> Fn { return tracer_stage_kernel<Form, R, SL>; };
     Fn fn = pick_scheme<Form>(s, pick);
-    hipLaunchKernelGGL(fn, dim3((inner + 255) / 256), dim3(256), 0, st, g, p, wtr, p.frx, p.fry);
+    hipLaunchKernelGGL(fn, dim3((unsigned)(g.strips * g.nspans * g.ntr)), dim3(kWave), 0, st, g, p);
     return hipGetLastError();
 }
 

@@ -78,10 +78,8 @@ hipError_t launch_stage1d_f32c(const Schemes& s, int kind, int reduce_dt, int xc
                                hipStream_t st, int virt = 0, int32_t faces = 0);
 
 // Tracer planes of a 2-D stage (p.frx / p.fry hold the stage's density fluxes).
-hipError_t launch_tracer_f64(const Schemes& s, const TracerGrid& g, const FormF64::Ptrs& p, double* wtr,
-                             hipStream_t st);
-hipError_t launch_tracer_f32c(const Schemes& s, const TracerGrid& g, const FormF32c::Ptrs& p, float* wtr,
-                              hipStream_t st);
+hipError_t launch_tracer_f64(const Schemes& s, const TracerGrid& g, const FormF64::Ptrs& p, hipStream_t st);
+hipError_t launch_tracer_f32c(const Schemes& s, const TracerGrid& g, const FormF32c::Ptrs& p, hipStream_t st);
 hipError_t launch_tracer_ghost_f64(const GhostGrid& g, int ntr, FormF64::Planes in, FormF64::Planes out,
                                    hipStream_t st);
 hipError_t launch_tracer_ghost_f32c(const GhostGrid& g, int ntr, FormF32c::Planes in, FormF32c::Planes out,
