@@ -103,7 +103,7 @@ struct FormF32c {
     struct Buf {
         __amdgpu_buffer_rsrc_t hi, lo;
     };
-    // 2-D grids with copy-type faces read ghost rows and columns from their
+    // the stages may read ghost cells from their
     // sources instead of filling them after every stage (StageGrid::virt)
     static constexpr bool kVirtualGhosts = true;
     static constexpr bool kHasFloors = true;  // positivity floors (floors_on)

@@ -37,7 +37,7 @@ struct FormF64 {
     struct Buf {
         __amdgpu_buffer_rsrc_t p;
     };
-    // grids with copy-type faces read ghost rows and columns from their
+    // the stages may read ghost cells from their
     // sources instead of filling them after every stage (StageGrid::virt)
     static constexpr bool kVirtualGhosts = true;
     static constexpr bool kHasFloors = false;  // positivity floors (floors_on)
