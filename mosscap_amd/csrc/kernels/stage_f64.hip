@@ -4,6 +4,15 @@
 #define MH_STAGE_WAVES_F64 1
 #endif
 #define MH_STAGE_WAVES_PER_EU MH_STAGE_WAVES_F64
+// The general WENO5-Z + HLLC instance takes 259 VGPRs (266 with mirrored
+// ghosts) when left alone, 3 to 10 more than let two wavefronts share a SIMD;
+// held to 256 it spills 1 (9) of them. A step with gravity then takes 893 us
+// instead of 1208 on 2048^2 periodic (953 instead of 1225 between walls) and
+// 253 instead of 314 on 1024^2. Launches of no more wavefronts than SIMDs
+// keep the one without spills: 640x480 with two tracers, stage 41.3 us against
+// 42.6. The other schemes fit 256 as they are.
+#define MH_STAGE_WAVES_EXTRAS 2
+#define MH_STAGE_WAVES_LONE 1
 // The raw Q^(s) of the stencil rows stays in registers for the combine (no
 // second load of row j) with WENO5-Z; the other schemes keep 3 waves per
 // SIMD without it (PPM + HLL: 154 VGPRs, 180 with it).

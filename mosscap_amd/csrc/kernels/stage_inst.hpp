@@ -14,6 +14,10 @@
 #ifndef MH_STAGE_WAVES_EXTRAS
 #define MH_STAGE_WAVES_EXTRAS MH_STAGE_WAVES_PER_EU
 #endif
+// ... where no two of its wavefronts share a SIMD (WENO5-Z + HLLC)
+#ifndef MH_STAGE_WAVES_LONE
+#define MH_STAGE_WAVES_LONE MH_STAGE_WAVES_EXTRAS
+#endif
 // ... and of the plain instance with the positivity floors
 #ifndef MH_STAGE_WAVES_FLOORS
 #define MH_STAGE_WAVES_FLOORS MH_STAGE_WAVES_PER_EU
@@ -21,11 +25,15 @@
 
 namespace mh {
 
-template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS, int Inst, bool Copies>
-__global__ __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(Inst == kStageExtras   ? MH_STAGE_WAVES_EXTRAS
-                                   : Inst == kStageFloors ? MH_STAGE_WAVES_FLOORS
-                                                          : MH_STAGE_WAVES_PER_EU)))
+// waves per SIMD that an instance of the 2-D stage must allow
+constexpr int stage_waves(int inst) {
+    return inst == kStageExtras ? MH_STAGE_WAVES_EXTRAS
+                                : inst == kStageFloors ? MH_STAGE_WAVES_FLOORS : MH_STAGE_WAVES_PER_EU;
+}
+
+template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS, int Inst, bool Copies,
+          int Waves = stage_waves(Inst)>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(Waves)))
 void stage2d_kernel(StageGrid g, typename Form::Ptrs p) {
     stage2d_march<Form, R, SL, RS, 2, Inst, Copies>(g, p);
 }
@@ -72,6 +80,11 @@ struct SolverPick {
             default: return stage2d_kernel<Form, R, SL, RiemannSolver::Hllc, Inst, Copies>;
         }
     }
+    // the general WENO5-Z + HLLC instance for wavefronts that have a SIMD each
+    template <bool Copies>
+    static Stage2dFn<Form> lone() {
+        return stage2d_kernel<Form, R, SL, RiemannSolver::Hllc, kStageExtras, Copies, MH_STAGE_WAVES_LONE>;
+    }
     static Stage1dFn<Form> one(RiemannSolver rs) {
         switch (rs) {
             case RiemannSolver::Rusanov: return stage1d_kernel<Form, R, SL, RiemannSolver::Rusanov>;
@@ -116,8 +129,13 @@ hipError_t launch_stage2d_impl(const Schemes& s, const StageGrid& g, const typen
     const bool extras = p.gravity != 0 || p.frx != nullptr || p.fry != nullptr || big;
     const bool floors = Form::floors_on(p);
     const bool copies = copy_stage_ghosts(g);
+    // no more wavefronts than SIMDs: none shares one
+    const bool lone = (int64_t)g.strips * g.nspans <= kSimds;
     auto pick = [&]<Reconstruction R, SlopeLimiter SL>() -> Stage2dFn<Form> {
         using P = SolverPick<Form, R, SL>;
+        if constexpr (R == Reconstruction::Weno5Z && MH_STAGE_WAVES_LONE != MH_STAGE_WAVES_EXTRAS) {
+            if (extras && lone && s.solver == RiemannSolver::Hllc) return copies ? P::template lone<true>() : P::template lone<false>();
+        }
         if (extras) return copies ? P::template two<kStageExtras, true>(s.solver) : P::template two<kStageExtras, false>(s.solver);
         if constexpr (Form::kHasFloors) {
             if (floors) return copies ? P::template two<kStageFloors, true>(s.solver) : P::template two<kStageFloors, false>(s.solver);

@@ -24,6 +24,8 @@ struct Schemes {
     TimeStepScheme stepper;
 };
 
+constexpr int kSimds = 1024;  // of the chip: 256 CUs of four
+
 // Number of marches that `rows` rows (or planes) are split into when `units`
 // wavefronts run side by side for each. A wavefront costs its rows plus a
 // prologue of `prologue` rows' worth, so fewer and longer marches do less
@@ -41,7 +43,6 @@ struct Schemes {
 // and 28 to 14 us (FP32C), at 512^2 from 44 to 32 and 31 to 21 us, at 1024^2
 // from 99 to 78 and 49 to 40 us; 2048^2 and up are unchanged to 1 %.
 inline int split_marches(int64_t units, int rows, double prologue, bool fp64) {
-    constexpr int kSimds = 1024;
     const int resident = fp64 ? 2 : 4;
     const double share64[] = {0.0, 1.18, 2.08}, share32[] = {0.0, 1.9, 2.4, 3.15, 4.0};  // of 1, 2, .. wavefronts
     const double* share = fp64 ? share64 : share32;
