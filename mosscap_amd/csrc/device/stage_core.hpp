@@ -523,11 +523,16 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
         }
 
         // 3-D: this row's z flux differences into registers now, so the
-        // load has the sweeps to arrive (without kDzLds)
+        // load has the sweeps to arrive (without kDzLds). Output lanes only:
+        // a ghost lane's c_ld is its source column, whose cache lines (one a
+        // variable and row) another strip reads (248x128x200 PPM + HLL step
+        // 1123 us with them, 1112 without; WENO5-Z + HLLC 1158 and 1143).
         T dzr[ND > 2 && !kDzLds ? NV : 1];
         if constexpr (ND > 2 && !kDzLds) {
+            if (out_lane) {
 #pragma unroll
-            for (int v = 0; v < NV; ++v) dzr[v] = p.dz3[v * plane + j * xc + c_ld];
+                for (int v = 0; v < NV; ++v) dzr[v] = p.dz3[v * plane + j * xc + c_ld];
+            }
         }
 
         // y sweep: cell j+1, face j+1
