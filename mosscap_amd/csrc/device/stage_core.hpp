@@ -527,12 +527,20 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
         // a ghost lane's c_ld is its source column, whose cache lines (one a
         // variable and row) another strip reads (248x128x200 PPM + HLL step
         // 1123 us with them, 1112 without; WENO5-Z + HLLC 1158 and 1143).
+        // In FP64 the branch costs registers, so every lane loads; the general
+        // WENO5-Z + HLLC instance, which is held to 256 VGPRs, loads them with
+        // its operands just before the combine instead: held across the sweeps
+        // they spill 24 registers more (66 against 42; 248x128x200 with
+        // gravity: step 3876 us against 3093, the other schemes 1 to 11 % faster
+        // with the early load).
+        constexpr bool kDzLate = !kDmaOps && sizeof(T) == 8 && R == Reconstruction::Weno5Z && RS == RiemannSolver::Hllc;
         T dzr[ND > 2 && !kDzLds ? NV : 1];
-        if constexpr (ND > 2 && !kDzLds) {
-            if (out_lane) {
+        auto load_dz = [&] {
 #pragma unroll
-                for (int v = 0; v < NV; ++v) dzr[v] = p.dz3[v * plane + j * xc + c_ld];
-            }
+            for (int v = 0; v < NV; ++v) dzr[v] = p.dz3[v * plane + j * xc + c_ld];
+        };
+        if constexpr (ND > 2 && !kDzLds && !kDzLate) {
+            if (sizeof(T) == 8 || out_lane) load_dz();
         }
 
         // y sweep: cell j+1, face j+1
@@ -593,6 +601,7 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
         }
         if (out_lane) {
             if constexpr (!Form::kEarlyOperands && !kDmaOps) load_operands();
+            if constexpr (ND > 2 && !kDzLds && kDzLate) load_dz();
             Raw qo[NV];
             T srcv[NV];
             if (Extras && p.gravity) {

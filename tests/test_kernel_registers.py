@@ -69,3 +69,10 @@ def test_fp64_general_instance_two_waves_per_simd(kernels, recon, solver, copies
     every = _instances(kernels, "stage2d_kernel", recon, solver, 2, copies)
     limiters = {"fog": 1, "muscl": 3, "ppm": 3, "weno5z": 1}[recon]
     assert sum(_waves(k) >= 2 for k in every) == limiters
+
+
+@pytest.mark.parametrize("copies", [True, False])
+def test_fp64_general_3d_march_spills(kernels, copies):
+    """Held to two wavefronts per SIMD, WENO5-Z + HLLC spills; no more than before ghosts were mirrored."""
+    (k,) = _instances(kernels, "stage3d_kernel", "weno5z", "hllc", True, copies)
+    assert _waves(k) >= 2 and k[".vgpr_spill_count"] <= 60
