@@ -2,9 +2,15 @@
 // form, built with -ffp-contract=fast-honor-pragmas like the 2-D unit. Five variables per
 // cell need more registers than the 2-D march: the plain instance is held to
 // at least three waves per SIMD (it takes 112 VGPRs, four waves), the one with
-// the gravity source to two.
+// the gravity source and the floors to two.
 #define MH_STAGE_WAVES_PER_EU 3
-#define MH_STAGE_WAVES_EXTRAS 2
+// FOG and PPM + Rusanov or HLL fit four and three without spills, which their
+// instances with mirrored ghosts exceed by a few registers when left alone
+// (FOG 134 VGPRs, PPM 175; 150x140x130 with gravity: FOG step 525 us, 382 so).
+#define MH_STAGE_WAVES_EXTRAS                                                 \
+    (R == Reconstruction::Fog && RS != RiemannSolver::Hll    ? 4              \
+     : R == Reconstruction::Ppm && RS != RiemannSolver::Hllc ? 3              \
+                                                             : 2)
 #ifndef MH_STAGE_QS_RING_F32C3
 #define MH_STAGE_QS_RING_F32C3 0
 #endif

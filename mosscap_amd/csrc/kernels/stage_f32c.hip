@@ -8,7 +8,10 @@
 #define MH_STAGE_WAVES_F32C 4
 #endif
 #define MH_STAGE_WAVES_PER_EU MH_STAGE_WAVES_F32C
-#define MH_STAGE_WAVES_EXTRAS 3
+// MUSCL + Rusanov fits four: left alone, its instance with mirrored ghosts takes
+// 129 VGPRs and three, one fewer than the division into spans counts on (2048^2
+// with gravity between walls: step 460 us, 315 so).
+#define MH_STAGE_WAVES_EXTRAS (R == Reconstruction::Muscl && RS == RiemannSolver::Rusanov ? 4 : 3)
 #define MH_STAGE_WAVES_FLOORS 4
 // The raw Q^(s) of the stencil rows stays in registers for the combine
 // (no second load of row j).

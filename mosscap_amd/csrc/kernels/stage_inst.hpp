@@ -5,18 +5,17 @@
 #include "../launch.hpp"
 #include "../device/tracer.hpp"
 
-// Occupancy target of the fused stage (waves per SIMD the register allocator
-// must allow); each form's translation unit sets its own value.
+// Occupancy targets of the fused stage (waves per SIMD the register allocator
+// must allow); each form's translation unit sets its own values, which may
+// depend on the instance's scheme (R, RS).
 #ifndef MH_STAGE_WAVES_PER_EU
 #define MH_STAGE_WAVES_PER_EU 1
 #endif
-// ... of the instance with the gravity source and tracer stores
+// ... of the instance with the gravity source and tracer stores (and, where
+// MH_STAGE_WAVES_LONE is set, of its WENO5-Z + HLLC scheme in launches of no
+// more wavefronts than SIMDs)
 #ifndef MH_STAGE_WAVES_EXTRAS
 #define MH_STAGE_WAVES_EXTRAS MH_STAGE_WAVES_PER_EU
-#endif
-// ... where no two of its wavefronts share a SIMD (WENO5-Z + HLLC)
-#ifndef MH_STAGE_WAVES_LONE
-#define MH_STAGE_WAVES_LONE MH_STAGE_WAVES_EXTRAS
 #endif
 // ... and of the plain instance with the positivity floors
 #ifndef MH_STAGE_WAVES_FLOORS
@@ -25,14 +24,14 @@
 
 namespace mh {
 
-// waves per SIMD that an instance of the 2-D stage must allow
+template <Reconstruction R, RiemannSolver RS>
 constexpr int stage_waves(int inst) {
     return inst == kStageExtras ? MH_STAGE_WAVES_EXTRAS
                                 : inst == kStageFloors ? MH_STAGE_WAVES_FLOORS : MH_STAGE_WAVES_PER_EU;
 }
 
 template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS, int Inst, bool Copies,
-          int Waves = stage_waves(Inst)>
+          int Waves = stage_waves<R, RS>(Inst)>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(Waves)))
 void stage2d_kernel(StageGrid g, typename Form::Ptrs p) {
     stage2d_march<Form, R, SL, RS, 2, Inst, Copies>(g, p);
@@ -80,11 +79,13 @@ struct SolverPick {
             default: return stage2d_kernel<Form, R, SL, RiemannSolver::Hllc, Inst, Copies>;
         }
     }
+#ifdef MH_STAGE_WAVES_LONE
     // the general WENO5-Z + HLLC instance for wavefronts that have a SIMD each
     template <bool Copies>
     static Stage2dFn<Form> lone() {
         return stage2d_kernel<Form, R, SL, RiemannSolver::Hllc, kStageExtras, Copies, MH_STAGE_WAVES_LONE>;
     }
+#endif
     static Stage1dFn<Form> one(RiemannSolver rs) {
         switch (rs) {
             case RiemannSolver::Rusanov: return stage1d_kernel<Form, R, SL, RiemannSolver::Rusanov>;
@@ -129,13 +130,15 @@ hipError_t launch_stage2d_impl(const Schemes& s, const StageGrid& g, const typen
     const bool extras = p.gravity != 0 || p.frx != nullptr || p.fry != nullptr || big;
     const bool floors = Form::floors_on(p);
     const bool copies = copy_stage_ghosts(g);
-    // no more wavefronts than SIMDs: none shares one
-    const bool lone = (int64_t)g.strips * g.nspans <= kSimds;
     auto pick = [&]<Reconstruction R, SlopeLimiter SL>() -> Stage2dFn<Form> {
         using P = SolverPick<Form, R, SL>;
-        if constexpr (R == Reconstruction::Weno5Z && MH_STAGE_WAVES_LONE != MH_STAGE_WAVES_EXTRAS) {
+#ifdef MH_STAGE_WAVES_LONE
+        if constexpr (R == Reconstruction::Weno5Z) {
+            // no more wavefronts than SIMDs: none shares one
+            const bool lone = (int64_t)g.strips * g.nspans <= kSimds;
             if (extras && lone && s.solver == RiemannSolver::Hllc) return copies ? P::template lone<true>() : P::template lone<false>();
         }
+#endif
         if (extras) return copies ? P::template two<kStageExtras, true>(s.solver) : P::template two<kStageExtras, false>(s.solver);
         if constexpr (Form::kHasFloors) {
             if (floors) return copies ? P::template two<kStageFloors, true>(s.solver) : P::template two<kStageFloors, false>(s.solver);
@@ -163,7 +166,7 @@ hipError_t launch_stage1d_impl(const Schemes& s, int kind, int reduce_dt, int xc
 #ifdef MH_STAGE3D_INSTANCES
 template <class Form, Reconstruction R, SlopeLimiter SL, RiemannSolver RS, bool Extras, bool Copies>
 __global__ __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(Extras ? MH_STAGE_WAVES_EXTRAS : MH_STAGE_WAVES_PER_EU)))
+__attribute__((amdgpu_waves_per_eu(stage_waves<R, RS>(Extras ? kStageExtras : kStagePlain))))
 void stage3d_kernel(StageGrid g, typename Form::Ptrs p) {
     stage2d_march<Form, R, SL, RS, 3, Extras ? kStageExtras : kStagePlain, Copies>(g, p);
 }

@@ -47,11 +47,11 @@ def kernels():
     return {k[".name"]: k for elf in _code_objects(blob) for k in _kernels(elf)}
 
 
-def _instances(kernels, name, recon, solver, *rest):
-    """FP64 instances of `name`, scheme enums as in the bindings, `rest` the further template arguments."""
+def _instances(kernels, name, recon, solver, *rest, form="7FormF64"):
+    """Instances of `name`, scheme enums as in the bindings, `rest` the further template arguments."""
     tail = "".join(f"Lb{int(r)}E" if isinstance(r, bool) else f"Li{r}E" for r in rest)
     found = [k for n, k in kernels.items()
-             if f"{name}INS_7FormF64" in n and f"ReconstructionE{M.RECONSTRUCTION[recon]}E" in n
+             if f"{name}INS_{form}" in n and f"ReconstructionE{M.RECONSTRUCTION[recon]}E" in n
              and f"RiemannSolverE{M.RIEMANN_SOLVER[solver]}E{tail}" in n]
     assert found, (name, recon, solver, rest)
     return found
@@ -76,3 +76,16 @@ def test_fp64_general_3d_march_spills(kernels, copies):
     """Held to two wavefronts per SIMD, WENO5-Z + HLLC spills; no more than before ghosts were mirrored."""
     (k,) = _instances(kernels, "stage3d_kernel", "weno5z", "hllc", True, copies)
     assert _waves(k) >= 2 and k[".vgpr_spill_count"] <= 60
+
+
+# the wavefronts per SIMD that the division into spans counts on (four) or that the scheme had
+@pytest.mark.parametrize("copies", [True, False])
+@pytest.mark.parametrize("name,recon,solver,waves", [("stage2d_kernel", "muscl", "rusanov", 4),
+                                                     ("stage3d_kernel", "fog", "rusanov", 4),
+                                                     ("stage3d_kernel", "fog", "hllc", 4),
+                                                     ("stage3d_kernel", "ppm", "rusanov", 3),
+                                                     ("stage3d_kernel", "ppm", "hll", 3)])
+def test_fp32c_general_instances(kernels, name, recon, solver, waves, copies):
+    every = _instances(kernels, name, recon, solver, 2 if name.startswith("stage2d") else True, copies,
+                       form="8FormF32c")
+    assert all(_waves(k) >= waves and k[".vgpr_spill_count"] == 0 for k in every)
