@@ -226,6 +226,11 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
     // where the lane loads (an output lane stores there too: its column is interior)
     const int c_ld = pl + ((kVirt && g.virt) ? source(min(c, g.xc - 1), g.nx, g.xf) : min(c, g.xc - 1));
     const bool x_flip = flips(min(c, g.xc - 1), g.nx, g.xf);
+    // where it loads z differences: a ghost lane's source column would cost a
+    // cache line per variable and row, which another strip reads (plain FP32C
+    // step on 248x128x200 periodic: PPM + HLL 1122 us with them, 1107 without;
+    // WENO5-Z + HLLC 1155 and 1144); the others load where they load the state
+    const int c_dz = Inst == kStagePlain && sizeof(T) == 4 ? pl + min(c, g.xc - 1) : c_ld;
     // source row of row r (wave-uniform)
     auto src_row = [&](int r) { return (kVirt && g.virt) ? source(r, g.ny, g.yf) : r; };
     const int xc = g.xc;
@@ -523,11 +528,7 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
         }
 
         // 3-D: this row's z flux differences into registers now, so the
-        // load has the sweeps to arrive (without kDzLds). Output lanes only:
-        // a ghost lane's c_ld is its source column, whose cache lines (one a
-        // variable and row) another strip reads (248x128x200 PPM + HLL step
-        // 1123 us with them, 1112 without; WENO5-Z + HLLC 1158 and 1143).
-        // In FP64 the branch costs registers, so every lane loads; the general
+        // load has the sweeps to arrive (without kDzLds). The general FP64
         // WENO5-Z + HLLC instance, which is held to 256 VGPRs, loads them with
         // its operands just before the combine instead: held across the sweeps
         // they spill 24 registers more (66 against 42; 248x128x200 with
@@ -537,11 +538,9 @@ __device__ inline void stage2d_march(const StageGrid& g, const typename Form::Pt
         T dzr[ND > 2 && !kDzLds ? NV : 1];
         auto load_dz = [&] {
 #pragma unroll
-            for (int v = 0; v < NV; ++v) dzr[v] = p.dz3[v * plane + j * xc + c_ld];
+            for (int v = 0; v < NV; ++v) dzr[v] = p.dz3[v * plane + j * xc + c_dz];
         };
-        if constexpr (ND > 2 && !kDzLds && !kDzLate) {
-            if (sizeof(T) == 8 || out_lane) load_dz();
-        }
+        if constexpr (ND > 2 && !kDzLds && !kDzLate) load_dz();
 
         // y sweep: cell j+1, face j+1
         T yl[NV], yr[NV], Gy[NV], dy[NV];
