@@ -153,10 +153,12 @@ int mh_adjoint_backward(mh_ctx* ctx, const double* lambda_final, double* lambda_
     DevPtr lamx{ctx->adj_scratch[0]}, acc{ctx->adj_scratch[1]}, cur{ctx->adj_scratch[2]}, nxt{ctx->adj_scratch[3]};
     std::vector<DevPtr> seg((size_t)every * ns);
     for (size_t k = 0; k < seg.size(); ++k) seg[k].p = ctx->adj_scratch[4 + k];
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    if (e == hipSuccess) e = hipEventCreate(&ev0);
-    if (e == hipSuccess) e = hipEventCreate(&ev1);
-    if (e == hipSuccess) e = hipEventRecord(ev0, ctx->stream);
+    // mh_adjoint_backward_ms: the last segment's recomputation (ev[0] to ev[1])
+    // and, the cotangent uploaded, the rest of the sweep (ev[2] to ev[3])
+    hipEvent_t ev[4] = {};
+    for (hipEvent_t& v : ev)
+        if (e == hipSuccess) e = hipEventCreate(&v);
+    if (e == hipSuccess) e = hipEventRecord(ev[0], ctx->stream);
     const int nseg = (int)ctx->ckpt.size();
     for (int sgi = nseg - 1; sgi >= 0 && e == hipSuccess; --sgi) {
         const int64_t n0 = (int64_t)sgi * every;
@@ -178,12 +180,15 @@ int mh_adjoint_backward(mh_ctx* ctx, const double* lambda_final, double* lambda_
             // the GPU recomputes the segment (and the result's pages are made
             // present while it runs the sweep: forward and reverse of 20 steps
             // at 512^2 8.42 -> 8.07 ms)
+            e = hipEventRecord(ev[1], ctx->stream);
             std::memcpy(ctx->adj_host, lambda_final, nv * sizeof(double));
-            e = hipMemcpyAsync(cur.p, ctx->adj_host, nv * sizeof(double), hipMemcpyHostToDevice, ctx->stream);
+            if (e == hipSuccess)
+                e = hipMemcpyAsync(cur.p, ctx->adj_host, nv * sizeof(double), hipMemcpyHostToDevice, ctx->stream);
             if (e == hipSuccess) e = launch_adjoint_axpby(g, 1.0, cur.p, 0.0, cur.p, ctx->stream);  // clear ghost entries
             // ... of the other cotangent buffer too: the line sweeps of a periodic
             // axis never write its ghost entries, which must read as zero
             if (e == hipSuccess) e = launch_adjoint_axpby(g, 1.0, nxt.p, 0.0, nxt.p, ctx->stream);
+            if (e == hipSuccess) e = hipEventRecord(ev[2], ctx->stream);
         }
         // reverse the segment's steps
         // cur holds the cotangent of step n's output; after the stages it holds
@@ -201,17 +206,18 @@ int mh_adjoint_backward(mh_ctx* ctx, const double* lambda_final, double* lambda_
             }
         }
     }
-    if (e == hipSuccess) e = hipEventRecord(ev1, ctx->stream);
+    if (e == hipSuccess) e = hipEventRecord(ev[3], ctx->stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(ctx->adj_host, cur.p, nv * sizeof(double), hipMemcpyDeviceToHost, ctx->stream);
     if (e == hipSuccess) populate_pages(lambda_initial, nv * sizeof(double));  // while the GPU runs the sweep
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e == hipSuccess) std::memcpy(lambda_initial, ctx->adj_host, nv * sizeof(double));
-    float ms = 0.0f;
-    if (e == hipSuccess) e = hipEventElapsedTime(&ms, ev0, ev1);
-    ctx->adj_bwd_ms = e == hipSuccess ? (double)ms : -1.0;
-    if (ev0) hipEventDestroy(ev0);
-    if (ev1) hipEventDestroy(ev1);
+    float before = 0.0f, after = 0.0f;
+    if (e == hipSuccess) e = hipEventElapsedTime(&before, ev[0], ev[1]);
+    if (e == hipSuccess) e = hipEventElapsedTime(&after, ev[2], ev[3]);
+    ctx->adj_bwd_ms = e == hipSuccess ? (double)before + (double)after : -1.0;
+    for (hipEvent_t v : ev)
+        if (v) hipEventDestroy(v);
     return e == hipSuccess ? MH_OK : ctx->hip_fail(e, "mh_adjoint_backward");
 }
 
