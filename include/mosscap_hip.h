@@ -138,9 +138,11 @@ int mh_stage(mh_ctx* ctx, int32_t stage, double dt);
  * state, except right after another mh_run, or an mh_time_step that followed
  * mh_compute_dt, whose last stage left the current state's maximum signal speed
  * behind (every other call that changes the state clears it); mh_compute_dt
- * uses it too. A caller that writes the state through
- * mh_device_state outside a user_bc hook calls mh_fill_bcs afterwards, as the
- * reference's setup does, which clears it too. */
+ * uses it too. Once mh_device_state has given out the state outside a user_bc
+ * hook, a caller may write it between calls, and every first dt comes from a
+ * CFL pass; such a caller calls mh_fill_bcs after a write, as the reference's
+ * setup does, or the next stage reads the ghosts as they were left (except
+ * periodic and zerograd ones of 2-D and 3-D grids without tracers). */
 int mh_run(mh_ctx* ctx, int64_t nsteps, double max_cfl, double* time, double max_time, double* prev_output_time,
            double delta, int32_t use_graph);
 

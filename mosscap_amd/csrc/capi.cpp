@@ -510,8 +510,9 @@ int mh_run(mh_ctx* ctx, int64_t nsteps, double max_cfl, double* time, double max
     hipError_t e = hipSetDevice(ctx->device);
     // Steady state: the previous mh_run's last stage left the max signal
     // speed of the current state in the CFL slots, so only the clock's
-    // fields are written; otherwise a CFL pass over the state fills them.
-    const bool keep_max = ctx->amax_valid;
+    // fields are written; otherwise, and where a caller may have written the
+    // state since, a CFL pass over the state fills them.
+    const bool keep_max = ctx->amax_valid && !ctx->exposed;
     ctx->forget_speed();
     ctx->dt_known = false;
     if (e == hipSuccess)
@@ -562,7 +563,7 @@ int mh_run(mh_ctx* ctx, int64_t nsteps, double max_cfl, double* time, double max
     if (e != hipSuccess) return ctx->hip_fail(e, "mh_run");
     const Clock h = *ctx->clock_host;
     if (const int rc = tab_check(ctx); rc != MH_OK) return rc;
-    ctx->amax_valid = true;
+    ctx->amax_valid = !ctx->exposed;
     *time = h.time;
     *prev_output_time = h.prev_output_time;
     ctx->time = h.time;

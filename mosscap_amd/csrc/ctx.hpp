@@ -91,7 +91,8 @@ struct mh_ctx {
     // stage folds the maximum
     bool fold_next = false;
     // the state's device pointers were given out (mh_device_state outside a
-    // hook): a caller may write it unseen, so mh_compute_dt always rescans
+    // hook): a caller may write it unseen, so mh_compute_dt and mh_run always
+    // rescan
     bool exposed = false;
     // step size in the device clock, when the host knows it
     bool dt_known = false;
