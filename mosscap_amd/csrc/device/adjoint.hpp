@@ -192,6 +192,13 @@ __host__ __device__ inline void weno5z_vjp(const double (&s)[5], double lL, doub
     ls[4] += la2 + lb2 + 2.0 * leL[2] - leR[0];
 }
 
+// cs = sqrt(gamma p / rho): dcs/drho = -cs/(2 rho) and dcs/dp = cs/(2p), so that
+// the cotangent lcs of cs adds -h/rho and h/p with h = lcs cs / 2. Without
+// pressure dcs/dp is infinite (and 0 lcs of it undefined), not 0/0.
+__host__ __device__ inline double sound_speed_dp(double cs, double lcs, double h, const Recip<double>& ip) {
+    return cs == 0.0 ? lcs * __builtin_inf() : ip.mul(h);
+}
+
 // Rusanov (Riemann.hpp:22-46), 2-D along Axis: accumulate J^T lf into lwL, lwR.
 template <int Axis>
 __host__ __device__ inline void rusanov_vjp2(double gamma, const double (&wL)[4], const double (&wR)[4],
@@ -246,12 +253,10 @@ __host__ __device__ inline void rusanov_vjp2(double gamma, const double (&wL)[4]
     for (int k = 0; k < 4; ++k) dq += lf[k] * (qR[k] - qL[k]);
     const double lc = -0.5 * dq;  // cotangent of max_c
     auto dcs = [&](const double (&w)[4], double cs, double (&o)[4]) {
-        // cs = sqrt(g p / rho): dcs/drho = -cs/(2 rho), dcs/dp = g / (2 rho cs)
         const double lcs = 0.5 * lc;
-        // = cs / (2p)
         const double h = 0.5 * lcs * cs;
         o[0] -= Recip<double>(w[0]).mul(h);
-        o[3] += Recip<double>(w[3]).mul(h);
+        o[3] += sound_speed_dp(cs, lcs, h, Recip<double>(w[3]));
         const double vn = w[IV];
         const double sg = vn > 0.0 ? 1.0 : (vn < 0.0 ? -1.0 : 0.0);
         o[IV] += lcs * sg;
@@ -438,11 +443,11 @@ __host__ __device__ inline void hllc_vjp2(double gamma, const double (&wL)[4], c
     gR[3] += igm1.mul(l_qRe);
     gR[1] += l_qRe * rR * wR[1];
     gR[2] += l_qRe * rR * wR[2];
-    // cs = sqrt(gamma*p/rho): dcs/dp = cs/(2p), dcs/drho = -cs/(2rho)
+    // cs = sqrt(gamma*p/rho)
     const double hL = 0.5 * l_csL * csL, hR = 0.5 * l_csR * csR;
-    gL[3] += ipL.mul(hL);
+    gL[3] += sound_speed_dp(csL, l_csL, hL, ipL);
     gL[0] -= irL.mul(hL);
-    gR[3] += ipR.mul(hR);
+    gR[3] += sound_speed_dp(csR, l_csR, hR, ipR);
     gR[0] -= irR.mul(hR);
     for (int k = 0; k < 4; ++k) {
         lwL[k] += gL[k];
