@@ -120,8 +120,8 @@ __host__ __device__ inline void cons_to_prim_vjp2(double gamma, const double (&q
 
 // WENO5-Z (Reconstruct.hpp:217-274): given the cotangents lL, lR of the
 // left/right face values of the cell, accumulate d(lL*wL + lR*wR)/ds into ls.
-// What decides a branch (the sign of beta0 - beta2) is computed as the forward
-// does; the rest multiplies by the five reciprocals of the cell's denominators
+// What decides a branch (the sign of beta0 - beta2) has the forward's bits (its
+// fmas multiply by powers of two); the rest multiplies by the five reciprocals of the cell's denominators
 // (12 divisions otherwise) and fuses its multiply-adds.
 struct WenoParts {
     double a[3], b[3], be[3];
@@ -134,7 +134,7 @@ __host__ __device__ inline WenoParts weno5z_parts(const double (&s)[5]) {
     const double a2 = s0 - 2.0 * sp1 + sp2, b2 = 3.0 * s0 - 4.0 * sp1 + sp2;
     return {{a0, a1, a2},
             {b0, b1, b2},
-            {c0 * a0 * a0 + c1 * b0 * b0, c0 * a1 * a1 + c1 * b1 * b1, c0 * a2 * a2 + c1 * b2 * b2}};
+            {c0 * (a0 * a0) + c1 * (b0 * b0), c0 * (a1 * a1) + c1 * (b1 * b1), c0 * (a2 * a2) + c1 * (b2 * b2)}};
 }
 __host__ __device__ inline void weno5z_vjp(const double (&s)[5], double lL, double lR, double (&ls)[5]) {
 #pragma clang fp contract(fast)
