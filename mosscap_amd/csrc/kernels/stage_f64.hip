@@ -3,7 +3,9 @@
 #ifndef MH_STAGE_WAVES_F64
 #define MH_STAGE_WAVES_F64 1
 #endif
-#define MH_STAGE_WAVES_PER_EU MH_STAGE_WAVES_F64
+// PPM + Rusanov fits three: left alone, its van Leer instance with mirrored ghosts
+// takes 171 VGPRs and two (2048^2 between walls: step 644 us, 599 so).
+#define MH_STAGE_WAVES_PER_EU (R == Reconstruction::Ppm && RS == RiemannSolver::Rusanov ? 3 : MH_STAGE_WAVES_F64)
 // The general WENO5-Z + HLLC instance takes 259 VGPRs (266 with mirrored
 // ghosts) when left alone, 3 to 10 more than let two wavefronts share a SIMD;
 // held to 256 it spills 1 (9) of them. A step with gravity then takes 893 us

@@ -89,3 +89,9 @@ def test_fp32c_general_instances(kernels, name, recon, solver, waves, copies):
     every = _instances(kernels, name, recon, solver, 2 if name.startswith("stage2d") else True, copies,
                        form="8FormF32c")
     assert all(_waves(k) >= waves and k[".vgpr_spill_count"] == 0 for k in every)
+
+
+@pytest.mark.parametrize("copies", [True, False])
+def test_fp64_plain_ppm_rusanov_three_waves_per_simd(kernels, copies):
+    every = _instances(kernels, "stage2d_kernel", "ppm", "rusanov", 0, copies)
+    assert len(every) == 3 and all(_waves(k) >= 3 for k in every)
