@@ -98,6 +98,7 @@ struct Arith<Dual<N>> {
         for (int k = 0; k < N; ++k) r.d[k] = a.d[k] / (2.0 * s);
         return r;
     }
+    __host__ __device__ static inline Dual<N> sqrt_speed(const Dual<N>& a) { return sqrt(a); }
     __host__ __device__ static inline Dual<N> sqrt_mid(const Dual<N>& a) { return sqrt(a); }
     static constexpr double weno_eps = 1e-36;
 };

@@ -52,9 +52,10 @@ __device__ inline double div_ieee(double a, double b) {
     const double q = as * r;
     return __builtin_amdgcn_div_fixup(__builtin_amdgcn_div_fmas(__builtin_fma(-bs, q, as), r, q, scaled), b, a);
 }
-// sqrt(x) for x zero, negative (NaN) or within 2^+-900: Goldschmidt's
-// iteration from the hardware 1/sqrt(x) and two residual corrections, without
-// the scaling that smaller arguments need.
+// sqrt(x) for x zero, negative (NaN) or above 2^-900 and finite (smaller ones
+// come out to 1e-14): Goldschmidt's iteration (Goldschmidt, "Applications of
+// division by convergence", MIT, 1964) from the hardware 1/sqrt(x) and two
+// residual corrections, without the scaling that smaller arguments need.
 __device__ inline double sqrt_plain(double x) {
     double y = __builtin_amdgcn_rsq(x);
     y = x == 0.0 ? 0x1p+500 : y;  // 0 * finite = 0 below instead of 0 * inf
@@ -65,10 +66,16 @@ __device__ inline double sqrt_plain(double x) {
     g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
     return __builtin_fma(__builtin_fma(-g, g, x), h, g);
 }
+// ... and infinity (inf * 0 above)
+__device__ inline double sqrt_inf(double x) {
+    const double g = sqrt_plain(x);
+    return x == __builtin_inf() ? x : g;
+}
 #else
 __host__ inline double div_plain(double a, double b) { return a / b; }
 __host__ inline double div_ieee(double a, double b) { return a / b; }
 __host__ inline double sqrt_plain(double x) { return __builtin_sqrt(x); }
+__host__ inline double sqrt_inf(double x) { return __builtin_sqrt(x); }
 #endif
 
 // A divisor used more than once.

@@ -33,8 +33,11 @@ struct Arith<double> {
     // correctly rounded divide and sqrt, matching glibc on the host (fast64.hpp)
     __host__ __device__ static inline double div(double a, double b) { return div_ieee(a, b); }
     __host__ __device__ static inline double sqrt(double a) { return __builtin_sqrt(a); }
-    // ... of an argument that is 0 or of moderate size (a speed squared, HLLC's star factor)
+    // ... of an argument that is 0 or finite: HLLC's star factor, a flux's sound speeds (an infinite
+    // one is no flux: it comes out as NaN)
     __host__ __device__ static inline double sqrt_mid(double a) { return sqrt_plain(a); }
+    // ... infinity too: the signal speed, where it stops the clock
+    __host__ __device__ static inline double sqrt_speed(double a) { return sqrt_inf(a); }
     static constexpr double weno_eps = 1e-36;  // Reconstruct.hpp:237-239
 };
 
@@ -43,6 +46,7 @@ struct Arith<float> {
     // Precision form: hardware reciprocal / sqrt (about 1 ulp).
     __device__ static inline float div(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
     __device__ static inline float sqrt(float a) { return __builtin_amdgcn_sqrtf(a); }
+    __device__ static inline float sqrt_speed(float a) { return sqrt(a); }
     __device__ static inline float sqrt_mid(float a) { return sqrt(a); }
     static constexpr float weno_eps = 1e-15f;  // single-precision value, Reconstruct.hpp:235-236
 };
@@ -88,11 +92,12 @@ __host__ __device__ inline EosT<float> make_eos<float>(double gamma) {
     return e;
 }
 
-// sound_speed, Eos.hpp:54-59
-template <int NumDim, typename T, typename WType>
+// sound_speed, Eos.hpp:54-59 (Infinite: also where it is)
+template <int NumDim, bool Infinite = false, typename T, typename WType>
 __host__ __device__ inline T sound_speed(const T gamma, const WType& w) {
     using P = Prim<NumDim>;
-    return Arith<T>::sqrt_mid(Arith<T>::div(gamma * w[P::Pres], w[P::Rho]));
+    const T c2 = Arith<T>::div(gamma * w[P::Pres], w[P::Rho]);
+    return Infinite ? Arith<T>::sqrt_speed(c2) : Arith<T>::sqrt_mid(c2);
 }
 
 // cons_to_prim, Eos.hpp:61-79
@@ -391,7 +396,7 @@ __host__ __device__ inline void riemann_flux(const EosT<T>& eos, const WL& wL, c
 template <int NumDim, typename T, typename WType>
 __host__ __device__ inline T signal_speed(const T gamma, const WType& w) {
     using P = Prim<NumDim>;
-    const T cs = sound_speed<NumDim>(gamma, w);
+    const T cs = sound_speed<NumDim, true>(gamma, w);
     T vel2 = square(w[P::Vx]);
     if constexpr (NumDim > 1) vel2 += square(w[P::Vy]);
     if constexpr (NumDim > 2) vel2 += square(w[P::Vz]);
