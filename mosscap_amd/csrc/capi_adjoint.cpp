@@ -155,9 +155,7 @@ int mh_adjoint_backward(mh_ctx* ctx, const double* lambda_final, double* lambda_
     for (size_t k = 0; k < seg.size(); ++k) seg[k].p = ctx->adj_scratch[4 + k];
     // mh_adjoint_backward_ms: the last segment's recomputation (ev[0] to ev[1])
     // and, the cotangent uploaded, the rest of the sweep (ev[2] to ev[3])
-    hipEvent_t ev[4] = {};
-    for (hipEvent_t& v : ev)
-        if (e == hipSuccess) e = hipEventCreate(&v);
+    const hipEvent_t* ev = ctx->adj_ev;
     if (e == hipSuccess) e = hipEventRecord(ev[0], ctx->stream);
     const int nseg = (int)ctx->ckpt.size();
     for (int sgi = nseg - 1; sgi >= 0 && e == hipSuccess; --sgi) {
@@ -216,8 +214,6 @@ int mh_adjoint_backward(mh_ctx* ctx, const double* lambda_final, double* lambda_
     if (e == hipSuccess) e = hipEventElapsedTime(&before, ev[0], ev[1]);
     if (e == hipSuccess) e = hipEventElapsedTime(&after, ev[2], ev[3]);
     ctx->adj_bwd_ms = e == hipSuccess ? (double)before + (double)after : -1.0;
-    for (hipEvent_t v : ev)
-        if (v) hipEventDestroy(v);
     return e == hipSuccess ? MH_OK : ctx->hip_fail(e, "mh_adjoint_backward");
 }
 

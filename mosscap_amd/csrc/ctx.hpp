@@ -394,9 +394,10 @@ struct mh_ctx {
     int adj_every = 0;
     double adj_bwd_ms = 0.0;  // device time of the last reverse sweep
     // reverse-sweep scratch kept between mh_adjoint_backward calls (nvals
-    // doubles each) and pinned host staging for its transfers
+    // doubles each), pinned host staging for its transfers and its events
     std::vector<double*> adj_scratch;
     double* adj_host = nullptr;
+    hipEvent_t adj_ev[4] = {};
     hipError_t adjoint_scratch(size_t nbuf) {
         hipError_t e = hipSuccess;
         if (adj_scratch.size() != nbuf) {
@@ -406,6 +407,8 @@ struct mh_ctx {
                 e = hipMalloc(&adj_scratch[k], (size_t)nvals * sizeof(double));
         }
         if (e == hipSuccess && !adj_host) e = hipHostMalloc(&adj_host, (size_t)nvals * sizeof(double));
+        for (hipEvent_t& v : adj_ev)
+            if (e == hipSuccess && !v) e = hipEventCreate(&v);
         if (e != hipSuccess) free_adjoint_scratch();
         return e;
     }
@@ -415,6 +418,10 @@ struct mh_ctx {
         adj_scratch.clear();
         if (adj_host) hipHostFree(adj_host);
         adj_host = nullptr;
+        for (hipEvent_t& v : adj_ev) {
+            if (v) hipEventDestroy(v);
+            v = nullptr;
+        }
     }
     void free_adjoint() {
         for (double* p : ckpt)
