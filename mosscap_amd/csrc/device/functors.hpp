@@ -205,8 +205,16 @@ __host__ __device__ inline void reconstruct_stencil(const S& s, T& wL, T& wR) {
         const T dw_0 = slope_limiter<sl>(s(0) - s(-1), s(1) - s(0));
         const T dw_p = slope_limiter<sl>(s(1) - s(0), s(2) - s(1));
         constexpr T sixth = T(1) / T(6);
-        T l = T(0.5) * (s(-1) + s(0)) - sixth * (dw_0 - dw_m);
-        T r = T(0.5) * (s(0) + s(1)) - sixth * (dw_p - dw_0);
+        // y - k x. In the precision form, whose units let multiply-adds fuse, this
+        // one always does: a k x - b y left to the compiler fused the one product
+        // or the other, and copies of one loop (ghosts filled or read from their
+        // sources) came out with other bits.
+        const auto minus = [](const T& y, T k, const T& x) -> T {
+            if constexpr (std::is_same_v<T, float>) return __builtin_fmaf(-k, x, y);
+            else return y - k * x;
+        };
+        T l = minus(T(0.5) * (s(-1) + s(0)), sixth, dw_0 - dw_m);
+        T r = minus(T(0.5) * (s(0) + s(1)), sixth, dw_p - dw_0);
         const T c = s(0);
         // sequential monotonicity fixes (not else-if), 204-214
         if ((r - c) * (c - l) <= T(0)) {
@@ -214,10 +222,10 @@ __host__ __device__ inline void reconstruct_stencil(const S& s, T& wL, T& wR) {
             r = c;
         }
         if (sabs(r - c) >= T(2) * sabs(l - c)) {
-            r = T(3) * c - T(2) * l;
+            r = minus(T(3) * c, T(2), l);
         }
         if (sabs(l - c) >= T(2) * sabs(r - c)) {
-            l = T(3) * c - T(2) * r;
+            l = minus(T(3) * c, T(2), r);
         }
         wL = l;
         wR = r;
