@@ -83,7 +83,7 @@ struct mh_batch {
             }
     }
 
-    // Periodic or zerograd faces: the persistent stage reads ghosts from
+    // Periodic or zerograd faces: the stage over all problems reads ghosts from
     // their source cells, so the stages of a step fill no ghosts and
     // mh_batch_run fills the final state's once (the ghosts would add nothing
     // to the per-problem CFL max: they copy interior values).
@@ -94,8 +94,8 @@ struct mh_batch {
         return copy_bc(bdry.xs) && copy_bc(bdry.xe);
     }
 
-    // one stage for every problem: persistent (mode 0) or one launch per problem (mode 1)
-    // fin, fin_cfl, fin_max_time: BatchGrid::fin and its arguments (persistent mode)
+    // one stage for every problem: one launch for all (mode 0) or one per problem (mode 1)
+    // fin, fin_cfl, fin_max_time: BatchGrid::fin and its arguments (mode 0)
     hipError_t stage(int mode, int in, int qn_k, int out, int kind, int reduce, int fin = 0, double fin_cfl = 0.0,
                      double fin_max_time = 0.0) {
         hipError_t e = hipSuccess;
@@ -162,7 +162,7 @@ struct mh_batch {
         }
         return in;
     }
-    // persistent steps of three or more stages (the second clears the CFL
+    // mode 0 steps of three or more stages (the second clears the CFL
     // maxima that only the last folds into)
     bool clock_in_stages(int mode) const { return mode == 0 && num_stages(sch.stepper) >= 3; }
     double graph_cfl = -1.0, graph_max_time = -1.0;  // the values the graphs were captured with

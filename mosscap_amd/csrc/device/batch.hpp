@@ -27,7 +27,7 @@ struct BatchGrid {
     int32_t ng, nitems, nprob, kind, reduce_dt;
     int32_t virt, faces;  // ghosts read from their sources (ghost_faces of the ends); no fill per stage
     // The step's per-problem clock work folded into its stages (graph-replayed
-    // persistent steps of three or more stages): 1 = this first stage takes
+    // steps over all problems of three or more stages): 1 = this first stage takes
     // each problem's dt from its CFL max and clock itself and the wave with
     // the problem's first segment stores it; 2 = that wave of this second
     // stage advances the problem's time and clears its CFL max. 0 = none.

@@ -5,8 +5,9 @@
 // the 2-D march turned to z), reconstructs every cell once, solves the
 // Riemann problem on each z face and stores the cell's flux difference
 // Fz_k - Fz_{k+1} (compute_recon_impl / compute_flux_impl with Axis = 2,
-// Hydro.cpp:55-166). The x-y march then runs once per interior z-plane and
-// adds that difference after the y one, the order of integrate_flux
+// Hydro.cpp:55-166). The x-y march then runs over every interior z-plane
+// (a wavefront's columns may end one plane and begin the next, march_columns)
+// and adds that difference after the y one, the order of integrate_flux
 // (TimeStepping.cpp:9-35). HBM traffic per cell and stage: the sweep reads
 // Q^(s) and writes NV values, the march reads Q^(s), Q^n and the NV values and
 // writes Q^(s+1).

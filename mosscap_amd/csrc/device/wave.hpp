@@ -8,9 +8,11 @@ namespace mh {
 
 constexpr int kWave = 64;
 
-// Orders LDS traffic between the lanes of one wavefront (the kernels that use
-// it run one wavefront per workgroup). LDS instructions of a wavefront execute
-// in issue order, so only compiler reordering has to be prevented.
+// Orders LDS traffic between the lanes of one wavefront, for LDS that no other
+// wavefront touches meanwhile (most kernels here run one per workgroup; the
+// adjoint's y sweep runs four, each on lines of its own between barriers). LDS
+// instructions of a wavefront execute in issue order, so only compiler
+// reordering has to be prevented.
 __device__ inline void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();

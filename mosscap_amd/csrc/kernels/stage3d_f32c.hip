@@ -1,4 +1,4 @@
-// 3-D stage kernels (z sweep + per-plane x-y march) of the compensated FP32
+// 3-D stage kernels (z sweep + x-y march) of the compensated FP32
 // form, built with -ffp-contract=fast-honor-pragmas like the 2-D unit. Five variables per
 // cell need more registers than the 2-D march: the plain instance is held to
 // at least three waves per SIMD (it takes 112 VGPRs, four waves), the one with

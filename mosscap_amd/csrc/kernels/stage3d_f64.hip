@@ -1,10 +1,12 @@
-// 3-D stage kernels (z sweep + per-plane x-y march) of the FP64 drop-in path,
+// 3-D stage kernels (z sweep + x-y march) of the FP64 drop-in path,
 // built with -ffp-contract=off like the 2-D units.
 // The 3-D march holds five variables per window row: it needs about 280
 // VGPRs unconstrained (one wavefront per SIMD); held to 256 (two), it spills
-// a few dwords. With two stencil rows in flight (loaded straight into LDS two
-// rows ahead) it spills 4 dwords instead of 25 and its stage runs 21 %
-// faster on the 256^3 blast than with one.
+// 17 of them (27 with mirrored ghosts; 5 with the compiler's divisions, whose
+// reciprocals live shorter, in a stage that took 1.1 to 1.3 times as long).
+// With two stencil rows in flight (loaded straight into LDS two rows ahead) the
+// march spilled 21 dwords fewer and its stage ran 21 % faster on the 256^3 blast
+// than with one.
 #ifndef MH_STAGE3D_WAVES_F64
 #define MH_STAGE3D_WAVES_F64 2
 #endif

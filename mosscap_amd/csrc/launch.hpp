@@ -37,7 +37,11 @@ constexpr int kSimds = 1024;  // of the chip: 256 CUs of four
 // (wavefronts that share a SIMD hide each other's latency: a lone FP32C row
 // takes 1.9 times its share of a full SIMD), plus a quarter of a wavefront
 // for the last round's uneven end.
-// Measured with every split from k = 1/2 to 16 on 256^2 to 4096^2 and 64^3
+// (Those are the WENO5-Z + HLLC marches' counts. Schemes that need fewer
+// registers hold more, the FP32C general instances three; over FOG to WENO5-Z,
+// every solver, both forms, 2-D and 3-D from 62^3 and 70x50 up, none is slower
+// than with the fixed minimum, but for 1 to 2 % of 186^3 in FP32C.)
+// Measured, WENO5-Z + HLLC, with every split from k = 1/2 to 16 on 256^2 to 4096^2 and 64^3
 // to 256^3: the pick is within 3 % of the best split, and against a fixed
 // minimum of 8 rows the WENO5-Z stage at 256^2 went from 42 to 18 us (FP64)
 // and 28 to 14 us (FP32C), at 512^2 from 44 to 32 and 31 to 21 us, at 1024^2
