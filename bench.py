@@ -525,10 +525,10 @@ def main(argv=None):
         "adjoint": adj,
         "roofline": {"bound": "hbm", "achieved": round(gbs32, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(gbs32 / HBM_PEAK_GBS, 4),
-                     # the plain instance (StageInst 0; named "false" before there were three)
+                     # the plain instance (StageInst 0) with copied ghosts
                      "traffic": measured_traffic("void mh::stage2d_kernel<mh::FormF32c, (mh::Reconstruction)3, "
                                                  "(mh::SlopeLimiter)1, (mh::RiemannSolver)2, ",
-                                                 ("0>(", "false>(")),
+                                                 ("0, true, ",)),
                      "kernel": "stage2d_kernel<FormF32c, Weno5Z, MC, HLLC, 0 (plain instance)>",
                      "avg_launch_ms": round(avg32, 4), "algorithmic_bytes_per_launch": int(bytes_per_launch)},
         "autotune": {"fp32c": tune32, "fp64": tune64},

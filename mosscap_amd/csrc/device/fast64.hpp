@@ -24,8 +24,8 @@
 //              1 + ind^2 = 1 whatever its last bits, so a tiny or zero tau
 //              needs no care.
 //
-// With them a WENO5-Z + HLLC stage issues 1656 VALU instructions per row of
-// the march instead of 2016; the KH step at 2048^2 takes 0.80 ms instead of
+// With them a WENO5-Z + HLLC stage issues 1572 VALU instructions per row of
+// the march instead of 1917; the KH step at 2048^2 takes 0.80 ms instead of
 // 0.93 and the one at 512^2 134 us instead of 156.
 #pragma once
 
